@@ -13,8 +13,10 @@
 //           so frames are deterministic -- no float atomics)
 // Path state is SoA in HBM indexed by the path's slot; queues hold slot ids
 // and are compacted per wave64 with a ballot + one atomic per wave.  Every
-// kernel fetches 64 items per wave from a device counter, so launches never
-// need the host to know queue lengths (no host round trip per stage).
+// kernel deals its queue over its waves from the length in a device counter,
+// so launches never need the host to know queue lengths (no host round trip
+// per stage).
+#include <algorithm>
 #include <mutex>
 #include <unordered_map>
 
@@ -30,47 +32,71 @@ constexpr int kBlock = 64;
 // ------------------------------------------------------------ wave helpers
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 
-// Items a wave takes per work-fetch atomic: kSub sub-batches of 64.  Every
+// Items a wave takes per work fetch: up to kSub sub-batches of 64.  Every
 // global counter here is touched by all waves of the grid, and device-scope
-// atomics on one address serialise across the chip, so each wave fetches
-// kSub * 64 items at once and publishes each output queue's survivors of all
-// sub-batches with one atomic.  Stages with little work per item take more
-// per fetch (ray generation 32 sub-batches, free flight 8), where the one
+// atomics on one address serialise across the chip, so a wave of a long queue
+// fetches kSub * 64 items at once and publishes each output queue's survivors
+// of all sub-batches with one atomic.  Stages with little work per item take
+// more per fetch (ray generation 32 sub-batches, free flight 8), where the one
 // counter's atomics would otherwise set the pace; the default of 4 measured
-// best for the others.
+// best for the others.  Short queues are dealt in smaller shares (Share).
 constexpr int kSub = 4;
+constexpr int kRaygenSub = 32, kMediumSub = 8;
+// Smallest share of the traversal kernels, whose lanes refill on their own:
+// with fewer rays than lanes a wave holds kTravGrain of them.
+constexpr int kTravGrain = 16;
 
-template <int kS = kSub>
-__device__ __forceinline__ uint32_t wave_fetch(uint32_t *work)
-{
-    uint32_t base = 0;
-    if (lane_id() == 0) base = atomicAdd(work, (uint32_t)(kBlock * kS));
-    return __shfl(base, 0);
-}
+// A wave's part of one slot's queue.  The first dealt() items of the queue
+// are dealt without atomics: the slot's home waves take grain() items each,
+// this wave [first, first_end).  The items past dealt() are fetched from the
+// slot's work counter, grain() at a time.  for_slots sets them; dealt and
+// grain are read once per fetch and wait in LDS (kShareWords words per wave),
+// where they cost the bodies no registers.
+constexpr int kShareWords = 5;
+// typed as LDS: a generic pointer would hold its 64-bit address in registers
+using LdsWord = volatile __attribute__((address_space(3))) uint32_t;
+struct Share {
+    LdsWord *w;
+    uint32_t first, first_end;
+    __device__ __forceinline__ uint32_t dealt() const { return __builtin_amdgcn_readfirstlane(w[0]); }
+    __device__ __forceinline__ uint32_t grain() const { return __builtin_amdgcn_readfirstlane(w[1]); }
+    // the next range of a queue of n items; false when none is left
+    __device__ __forceinline__ bool fetch(uint32_t *work, uint32_t n, uint32_t &cur, uint32_t &end) const
+    {
+        const uint32_t d = dealt();
+        if (d >= n) return false;
+        const uint32_t g = grain();
+        uint32_t got = 0;
+        if (__lane_id() == 0) got = atomicAdd(work, g);
+        const uint32_t base = d + (uint32_t)__builtin_amdgcn_readfirstlane(got);
+        if (base >= n) return false;
+        cur = base;
+        end = min(base + g, n);
+        return true;
+    }
+};
 
 // Persistent loop over n items (one wave per block): body(i, p, out) handles
 // item i < n, sets p (the path slot it appends) and out[q] for each output
-// queue q.  Survivors of a fetch's sub-batches are staged in LDS and then
-// published with one atomic per queue and a coalesced copy.
+// queue q.  Survivors of a fetch's sub-batches (at most kS) are staged in LDS and then published with one atomic per queue and
+// a coalesced copy.
 template <int kQueues, int kS = kSub, typename Body>
-__device__ __forceinline__ void run_items(uint32_t *fetch, uint32_t n, uint32_t *const *counters,
+__device__ __forceinline__ void run_items(const Share &share, uint32_t *fetch, uint32_t n, uint32_t *const *counters,
                                           uint32_t *const *queues, Body &&body)
 {
     constexpr int kQ = kQueues > 0 ? kQueues : 1;
     __shared__ uint32_t stage[kQ * kS * kBlock];
     const uint64_t below = (1ull << lane_id()) - 1ull;
+    uint32_t base = share.first, end = share.first_end;
     for (;;) {
-        const uint32_t base = wave_fetch<kS>(fetch);
-        if (base >= n) break;
+        if (base >= end && !share.fetch(fetch, n, base, end)) break;
         uint32_t filled[kQ] = {};
 #pragma unroll 1
-        for (int k = 0; k < kS; ++k) {
-            const uint32_t first = base + (uint32_t)k * kBlock;
-            if (first >= n) break;
-            const uint32_t i = first + lane_id();
+        for (; base < end; base += kBlock) {
+            const uint32_t i = base + lane_id();
             uint32_t p = 0;
             bool out[kQ] = {};
-            if (i < n) body(i, p, out);
+            if (i < end) body(i, p, out);
             static_for<0, kQueues>([&](auto Q) {
                 const uint64_t m = __ballot(out[Q()]);
                 if (out[Q()]) stage[Q() * kS * kBlock + filled[Q()] + (uint32_t)__popcll(m & below)] = p;
@@ -98,7 +124,8 @@ __device__ __forceinline__ void run_items(uint32_t *fetch, uint32_t n, uint32_t 
 // kRefillLanes lanes are done.  Ray lengths vary by orders of magnitude, so a
 // wave that waited for its slowest ray would run most of its steps with few
 // lanes active.  refill() hands the wave's idle lanes the next items of its
-// fetched range [cur, end), fetching kSub * 64 more as the range runs dry; it
+// range [cur, end), which starts as its dealt share and is fetched from the
+// work counter as it runs dry; it
 // returns true on the lanes that took item *item.  Refilling at 32 (extend)
 // and 16 (shadow) idle lanes measured fastest on the interior frame (extend:
 // 16, 24, 28, 40 and 48 were 1-13 % slower; shadow: 8, 24 and 32 were
@@ -106,24 +133,24 @@ __device__ __forceinline__ void run_items(uint32_t *fetch, uint32_t n, uint32_t 
 constexpr int kLaneIdle = 3;  // no ray (beside kTravContinue/Hit/Miss/Overflow)
 template <int kRefillLanes>
 struct RefillRange {
+    const Share &share;
     uint32_t *work;
     uint32_t n;
     uint32_t cur, end;
-    bool more;  // the work counter may hold items
+    bool more;  // the range or the work counter may hold items
+    __device__ __forceinline__ RefillRange(const Share &s, uint32_t *w, uint32_t count)
+        : share(s), work(w), n(count), cur(s.first), end(s.first_end), more(s.first < s.first_end || s.dealt() < count)
+    {
+    }
     __device__ __forceinline__ bool refill(bool idle_lane, uint32_t &item)
     {
         const uint64_t below = (1ull << lane_id()) - 1ull;
         bool took = false;
         uint64_t idle = __ballot(idle_lane);
         while (idle && more) {
-            if (cur >= end) {
-                const uint32_t base = wave_fetch(work);
-                if (base >= n) {
-                    more = false;
-                    break;
-                }
-                cur = base;
-                end = base + (uint32_t)(kBlock * kSub) < n ? base + (uint32_t)(kBlock * kSub) : n;
+            if (cur >= end && !share.fetch(work, n, cur, end)) {
+                more = false;
+                break;
             }
             const uint32_t take = min((uint32_t)__popcll(idle), end - cur);
             if (idle_lane && !took) {
@@ -136,6 +163,8 @@ struct RefillRange {
             cur += take;
             idle = __ballot(idle_lane && !took);
         }
+        // a queue dealt in full has nothing to fetch
+        if (more && cur >= end && share.dealt() >= n) more = false;
         return took;
     }
     // lanes to wait for before the next refill: all of them once the counter
@@ -280,44 +309,83 @@ __device__ __forceinline__ uint32_t pass_counter(const FrameSlot &f, uint32_t pa
 {
     return f.prm.counters[pass * kCtrStride + k];
 }
-
-// the work counter has passed the item count: nothing left to fetch
-__device__ __forceinline__ bool work_drained(const uint32_t *work, uint32_t n)
+__device__ __forceinline__ uint32_t *pass_work(const FrameSlot &f, uint32_t pass, uint32_t k)
 {
-    return __hip_atomic_load(work, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= n;
-}
-__device__ __forceinline__ bool pass_drained(const FrameSlot &f, uint32_t pass, uint32_t work, uint32_t count)
-{
-    const uint32_t *c = f.prm.counters + pass * kCtrStride;
-    return work_drained(c + work, c[count]);
+    return f.prm.counters + pass * kCtrStride + k;
 }
 
-template <typename Count, typename Drained, typename Body>
-__device__ __forceinline__ void for_slots(const FrameSlot *__restrict__ fs, uint32_t nfs, Count count,
-                                          Drained drained, Body body)
+// Runs body(f, share) for the slots this wave works on: its home slot first,
+// then the others.  count(f): the items queued in slot f; work(f): its work
+// counter.  A launch's items are dealt in shares of `grain`:
+//   * kMaxGrain when every wave of the grid gets that many: long queues, whose
+//     fetch atomics (tens of ns each on one address, one after another across
+//     the chip) would set the pace in smaller shares;
+//   * down to kMinGrain otherwise, so that a short queue is spread over all
+//     the waves the GPU holds: a wave's items run one sub-batch after another,
+//     each a chain of dependent loads, and with shares of kMaxGrain a
+//     65536-path launch would occupy 256 of 1024 SIMDs for four such chains.
+// The first share of each home wave is dealt by its index, so a queue that
+// one round of shares covers takes no atomics at all; waves without a share
+// leave at once.  Measured against shares of kMaxGrain from one counter:
+// Cornell 256x256 at 1 spp 6.9 -> 3.1 ms, its 512x512 smoke at 16 spp (23
+// passes, the last of them short) 49 -> 40 ms, the interior at 1080p and 1 spp
+// 27.7 -> 24.1 ms, at 64 spp 958 -> 950 ms.
+template <uint32_t kMinGrain, uint32_t kMaxGrain, typename Count, typename Work, typename Body>
+__device__ __forceinline__ void for_slots(const FrameSlot *__restrict__ fs, uint32_t nfs, Count count, Work work,
+                                          Body body)
 {
-    uint32_t total = 0;
-    for (uint32_t s = 0; s < nfs; ++s) total += count(fs[s]);
-    if (total == 0) return;
-    // waves beyond one per fetch of kSub * 64 items would find the stage
-    // dry: they leave without touching its work counter (whose atomics
-    // queue up behind each other), and the rest take every item
-    if ((uint64_t)blockIdx.x * (uint64_t)(kBlock * kSub) >= (uint64_t)total) return;
-    const uint32_t target = (uint32_t)(((uint64_t)blockIdx.x * total) / gridDim.x);
+    // words of Share, then what the next slot's deal needs: kept out of
+    // registers while a body runs
+    __shared__ uint32_t words[kShareWords];
+    LdsWord *w = (LdsWord *)words;
+    const uint32_t me = blockIdx.x;
     uint32_t home = 0;
-    for (uint32_t s = 0, acc = 0; s < nfs; ++s) {
-        acc += count(fs[s]);
-        if (acc > target) {
-            home = s;
-            break;
+    {
+        uint32_t total = 0;
+        for (uint32_t s = 0; s < nfs; ++s) total += count(fs[s]);
+        if (total == 0) return;
+        const uint32_t per = total / gridDim.x;
+        const uint32_t grain = per >= kMaxGrain ? kMaxGrain : per <= kMinGrain ? kMinGrain : per / kMinGrain * kMinGrain;
+        const uint32_t waves = min((total + grain - 1) / grain, gridDim.x);
+        if (me >= waves) return;
+        // wave w's home is the slot whose items hold item floor(w * total / waves)
+        uint32_t before = 0;
+        if (nfs > 1) {
+            const uint32_t target = (uint32_t)(((uint64_t)me * total) / waves);
+            for (uint32_t c; home + 1 < nfs && before + (c = count(fs[home])) <= target; ++home) before += c;
         }
+        w[1] = grain;
+        w[2] = total;
+        w[3] = waves;
+        w[4] = before;
     }
     for (uint32_t j = 0; j < nfs; ++j) {
-        uint32_t s = home + j;
-        s = __builtin_amdgcn_readfirstlane(s >= nfs ? s - nfs : s);
+        const uint32_t s = __builtin_amdgcn_readfirstlane(home + j >= nfs ? home + j - nfs : home + j);
         const FrameSlot &f = fs[s];
-        if (count(f) == 0 || drained(f)) continue;
-        body(f);
+        const uint32_t n = count(f);
+        const uint32_t before = s == 0 ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane(w[4]);
+        w[4] = before + n;
+        if (n == 0) continue;
+        const uint32_t grain = __builtin_amdgcn_readfirstlane(w[1]);
+        const uint32_t waves = __builtin_amdgcn_readfirstlane(w[3]);
+        // home waves of slot s: ceil(before * waves / total) up to
+        // ceil((before + n) * waves / total)
+        uint32_t w0 = 0, w1 = waves;
+        if (nfs > 1) {
+            const uint32_t total = __builtin_amdgcn_readfirstlane(w[2]);
+            w0 = (uint32_t)(((uint64_t)before * waves + total - 1) / total);
+            w1 = (uint32_t)(((uint64_t)(before + n) * waves + total - 1) / total);
+        }
+        const uint32_t dealt = (uint32_t)min((uint64_t)(w1 - w0) * grain, (uint64_t)n);
+        w[0] = dealt;
+        Share share{w, 0, 0};
+        if (j == 0) {
+            share.first = min((me - w0) * grain, n);
+            share.first_end = min(share.first + grain, n);
+        } else if (dealt >= n || dealt + __hip_atomic_load(work(f), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= n) {
+            continue;  // nothing left to fetch
+        }
+        body(f, share);
     }
 }
 
@@ -421,12 +489,14 @@ __device__ __forceinline__ f3 light_clamp(const ymrt_render_settings &rs, f3 c, 
 }
 
 // ------------------------------------------------------------ raygen
-__device__ __forceinline__ void raygen_body(const DevScene &sc, const PtParams &prm, const PathState &ps)
+__device__ __forceinline__ void raygen_body(const DevScene &sc, const PtParams &prm, const PathState &ps,
+                                            const Share &share)
 {
     uint32_t *cnt = prm.counters;  // pass 0 slots
     uint32_t *const ctrs[1] = {cnt + kCtrActive};
     uint32_t *const qs[1] = {ps.queue[0]};
-    run_items<1, 32>(cnt + kCtrWorkRaygen, prm.chunk_paths, ctrs, qs, [&](uint32_t p, uint32_t &slot, bool(&out)[1]) {
+    run_items<1, kRaygenSub>(share, cnt + kCtrWorkRaygen, prm.chunk_paths, ctrs, qs,
+                             [&](uint32_t p, uint32_t &slot, bool(&out)[1]) {
         slot = p;
         ps.flag[p] = 0;
         {
@@ -485,10 +555,10 @@ __device__ __forceinline__ void raygen_body(const DevScene &sc, const PtParams &
 
 __global__ __launch_bounds__(kBlock) void k_raygen_m(const FrameSlot *__restrict__ fs, uint32_t nfs)
 {
-    for_slots(
+    for_slots<kBlock, kBlock * kRaygenSub>(
         fs, nfs, [](const FrameSlot &f) { return f.prm.chunk_paths; },
-        [](const FrameSlot &f) { return work_drained(f.prm.counters + kCtrWorkRaygen, f.prm.chunk_paths); },
-        [](const FrameSlot &f) { raygen_body(f.sc, f.prm, f.ps); });
+        [](const FrameSlot &f) { return f.prm.counters + kCtrWorkRaygen; },
+        [](const FrameSlot &f, const Share &share) { raygen_body(f.sc, f.prm, f.ps, share); });
 }
 
 
@@ -503,7 +573,8 @@ __global__ __launch_bounds__(kBlock) void k_raygen_m(const FrameSlot *__restrict
 // (RefillRange).
 
 template <bool kNearby, bool kMedia, bool kSphere, int kStack>
-__device__ __forceinline__ void extend_body(const DevScene &sc, const PtParams &prm, const PathState &ps, uint32_t pass)
+__device__ __forceinline__ void extend_body(const DevScene &sc, const PtParams &prm, const PathState &ps, uint32_t pass,
+                                            const Share &share)
 {
     __shared__ uint32_t stack[kStackWindow * kBlock];
     __shared__ uint32_t nbp[(kNearby ? kNearbyCap : 1) * kBlock];
@@ -517,7 +588,7 @@ __device__ __forceinline__ void extend_body(const DevScene &sc, const PtParams &
     const ymrt_render_settings &rs = prm.rs;
     uint32_t rays = 0, cam_rays = 0;
     TraceCounters tc{0, 0};
-    RefillRange<32> rr{cnt + kCtrWorkExtend, cnt[kCtrActive], 0u, 0u, true};
+    RefillRange<32> rr(share, cnt + kCtrWorkExtend, cnt[kCtrActive]);
 
     Traversal<kModeAll, false, kNearby, true, kSphere, kStack> tv;
     uint32_t p = 0;
@@ -615,10 +686,12 @@ __device__ __forceinline__ void extend_body(const DevScene &sc, const PtParams &
 template <bool kNearby, bool kMedia, bool kSphere, int kStack>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kSphere ? 1 : 4))) void k_extend_m(const FrameSlot *__restrict__ fs, uint32_t nfs, uint32_t pass)
 {
-    for_slots(
+    for_slots<kTravGrain, kBlock * kSub>(
         fs, nfs, [&](const FrameSlot &f) { return pass_counter(f, pass, kCtrActive); },
-        [&](const FrameSlot &f) { return pass_drained(f, pass, kCtrWorkExtend, kCtrActive); },
-        [&](const FrameSlot &f) { extend_body<kNearby, kMedia, kSphere, kStack>(f.sc, f.prm, f.ps, pass); });
+        [&](const FrameSlot &f) { return pass_work(f, pass, kCtrWorkExtend); },
+        [&](const FrameSlot &f, const Share &share) {
+            extend_body<kNearby, kMedia, kSphere, kStack>(f.sc, f.prm, f.ps, pass, share);
+        });
 }
 
 
@@ -811,14 +884,15 @@ __global__ __launch_bounds__(kCompactThreads) void k_compact_scatter_m(const Fra
 // to 5 waves per SIMD (96 VGPRs, no spills): it waits on memory most of the
 // time, and the fifth wave measured 1.5 % faster than four.
 template <int kHet, bool kAdj = false>
-__device__ __forceinline__ void medium_body(const DevScene &sc, const PtParams &prm, const PathState &ps, uint32_t pass)
+__device__ __forceinline__ void medium_body(const DevScene &sc, const PtParams &prm, const PathState &ps, uint32_t pass,
+                                            const Share &share)
 {
     constexpr bool kGrid = kHet > 0;
     __shared__ float tex_stk[kHet == 2 ? kTexStack * 3 * kBlock : 1];
     uint32_t *cnt = prm.counters + pass * kCtrStride;
     const uint32_t n = cnt[kCtrMedium];
     const ymrt_render_settings &rs = prm.rs;
-    run_items<0, 8>(cnt + kCtrWorkMedium, n, nullptr, nullptr, [&](uint32_t i, uint32_t &p, bool(&)[1]) {
+    run_items<0, kMediumSub>(share, cnt + kCtrWorkMedium, n, nullptr, nullptr, [&](uint32_t i, uint32_t &p, bool(&)[1]) {
         {
             p = ps.q_medium[i];
             const uint4 ha = ps.hit_a[p];
@@ -884,10 +958,10 @@ __device__ __forceinline__ void medium_body(const DevScene &sc, const PtParams &
 template <int kHet, bool kAdj = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kHet ? 1 : 5))) void k_medium_m(const FrameSlot *__restrict__ fs, uint32_t nfs, uint32_t pass)
 {
-    for_slots(
+    for_slots<kBlock, kBlock * kMediumSub>(
         fs, nfs, [&](const FrameSlot &f) { return pass_counter(f, pass, kCtrMedium); },
-        [&](const FrameSlot &f) { return pass_drained(f, pass, kCtrWorkMedium, kCtrMedium); },
-        [&](const FrameSlot &f) { medium_body<kHet, kAdj>(f.sc, f.prm, f.ps, pass); });
+        [&](const FrameSlot &f) { return pass_work(f, pass, kCtrWorkMedium); },
+        [&](const FrameSlot &f, const Share &share) { medium_body<kHet, kAdj>(f.sc, f.prm, f.ps, pass, share); });
 }
 
 
@@ -969,7 +1043,8 @@ __device__ __forceinline__ float shadow_tmax(f3 pos, f3 ldir, f3 lpos, f3 lerr, 
 // kAdj: the adjoint's replay pass (surface vertices): albedo, texel and
 // roughness gradient events.
 template <bool kVolume, bool kGraph, uint32_t kClass = kMatGeneral, bool kAdj = false>
-__device__ __forceinline__ void shade_body(const DevScene &sc, const PtParams &prm, const PathState &ps, uint32_t pass)
+__device__ __forceinline__ void shade_body(const DevScene &sc, const PtParams &prm, const PathState &ps, uint32_t pass,
+                                           const Share &share)
 {
     __shared__ float tex_stk[(kVolume || !kGraph) ? 1 : kTexStack * 3 * kBlock];
     __shared__ float adj_lds[kAdj ? kAdjLds : 1];
@@ -987,7 +1062,7 @@ __device__ __forceinline__ void shade_body(const DevScene &sc, const PtParams &p
     constexpr uint32_t kLobes = kDiffuse ? 1u << kSlotDiffuse
                                 : kMetal ? (1u << kSlotMetal) | (1u << kSlotDiffuse)
                                          : 0u;
-    run_items<2>(cnt + (kVolume     ? kCtrWorkShadeVol
+    run_items<2>(share, cnt + (kVolume     ? kCtrWorkShadeVol
                         : kDiffuse ? kCtrWorkShadeDiffuse
                         : kMetal   ? kCtrWorkShadeMetal
                                    : kCtrWorkShade),
@@ -1414,10 +1489,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kGraph ?
                                 : kClass == kMatMetal ? kCtrHitMetal : kCtrHit;
     constexpr uint32_t kWork = kVolume ? kCtrWorkShadeVol : kClass == kMatDiffuse ? kCtrWorkShadeDiffuse
                                : kClass == kMatMetal ? kCtrWorkShadeMetal : kCtrWorkShade;
-    for_slots(
+    for_slots<kBlock, kBlock * kSub>(
         fs, nfs, [&](const FrameSlot &f) { return pass_counter(f, pass, kQueue); },
-        [&](const FrameSlot &f) { return pass_drained(f, pass, kWork, kQueue); },
-        [&](const FrameSlot &f) { shade_body<kVolume, kGraph, kClass, kAdj>(f.sc, f.prm, f.ps, pass); });
+        [&](const FrameSlot &f) { return pass_work(f, pass, kWork); },
+        [&](const FrameSlot &f, const Share &share) {
+            shade_body<kVolume, kGraph, kClass, kAdj>(f.sc, f.prm, f.ps, pass, share);
+        });
 }
 
 
@@ -1491,7 +1568,8 @@ __device__ __forceinline__ void shadow_finish(const PtParams &prm, const PathSta
 // paths with an unoccluded ray go on to k_transmit for the transmittance along
 // it; the others are finished here.
 template <bool kMedia, bool kSphere, int kStack, bool kAdj = false>
-__device__ __forceinline__ void shadow_body(const DevScene &sc, const PtParams &prm, const PathState &ps, uint32_t pass)
+__device__ __forceinline__ void shadow_body(const DevScene &sc, const PtParams &prm, const PathState &ps, uint32_t pass,
+                                            const Share &share)
 {
     __shared__ uint32_t stack[kStackWindow * kBlock];
     __shared__ float pre_park[kPreSlots * kBlock];
@@ -1504,7 +1582,7 @@ __device__ __forceinline__ void shadow_body(const DevScene &sc, const PtParams &
                                                ps.spill_threads, blockIdx.x * kBlock + threadIdx.x, pre_park};
     uint32_t nsh = 0;
     TraceCounters tc{0, 0};
-    RefillRange<16> rr{cnt + kCtrWorkShadow, cnt[kCtrShadow], 0u, 0u, true};
+    RefillRange<16> rr(share, cnt + kCtrWorkShadow, cnt[kCtrShadow]);
 
     // one lane walks its path's recorded rays (slots k) in order
     Traversal<kModeSkipBoundary, true, false, true, kSphere, kStack> tv;
@@ -1570,10 +1648,12 @@ __device__ __forceinline__ void shadow_body(const DevScene &sc, const PtParams &
 template <bool kMedia, bool kSphere, int kStack, bool kAdj = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_shadow_m(const FrameSlot *__restrict__ fs, uint32_t nfs, uint32_t pass)
 {
-    for_slots(
+    for_slots<kTravGrain, kBlock * kSub>(
         fs, nfs, [&](const FrameSlot &f) { return pass_counter(f, pass, kCtrShadow); },
-        [&](const FrameSlot &f) { return pass_drained(f, pass, kCtrWorkShadow, kCtrShadow); },
-        [&](const FrameSlot &f) { shadow_body<kMedia, kSphere, kStack, kAdj>(f.sc, f.prm, f.ps, pass); });
+        [&](const FrameSlot &f) { return pass_work(f, pass, kCtrWorkShadow); },
+        [&](const FrameSlot &f, const Share &share) {
+            shadow_body<kMedia, kSphere, kStack, kAdj>(f.sc, f.prm, f.ps, pass, share);
+        });
 }
 
 
@@ -1587,7 +1667,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // events, found by walking the ray a second time with the same random
 // numbers once its deposit is known.
 template <bool kSphere, int kStack, int kHet, bool kAdj = false>
-__device__ __forceinline__ void transmit_body(const DevScene &sc, const PtParams &prm, const PathState &ps, uint32_t pass)
+__device__ __forceinline__ void transmit_body(const DevScene &sc, const PtParams &prm, const PathState &ps, uint32_t pass,
+                                              const Share &share)
 {
     __shared__ float tex_stk[kHet == 2 ? kTexStack * 3 * kBlock : 1];
     __shared__ uint32_t stack[kStackWindow * kBlock];
@@ -1604,7 +1685,7 @@ __device__ __forceinline__ void transmit_body(const DevScene &sc, const PtParams
     __shared__ float adj_lds[kAdj ? kAdjLds : 1];
     AdjSums<kAdj> sums{adj_lds, &prm.adj};
     sums.begin();
-    run_items<0>(cnt + kCtrWorkTransmit, n, nullptr, nullptr, [&](uint32_t i, uint32_t &slot, bool(&)[1]) {
+    run_items<0>(share, cnt + kCtrWorkTransmit, n, nullptr, nullptr, [&](uint32_t i, uint32_t &slot, bool(&)[1]) {
         {
             const uint32_t p = ps.q_transmit[i];
             slot = p;
@@ -1727,10 +1808,12 @@ __device__ __forceinline__ void transmit_body(const DevScene &sc, const PtParams
 template <bool kSphere, int kStack, int kHet, bool kAdj = false>
 __global__ __launch_bounds__(kBlock) void k_transmit_m(const FrameSlot *__restrict__ fs, uint32_t nfs, uint32_t pass)
 {
-    for_slots(
+    for_slots<kBlock, kBlock * kSub>(
         fs, nfs, [&](const FrameSlot &f) { return pass_counter(f, pass, kCtrTransmit); },
-        [&](const FrameSlot &f) { return pass_drained(f, pass, kCtrWorkTransmit, kCtrTransmit); },
-        [&](const FrameSlot &f) { transmit_body<kSphere, kStack, kHet, kAdj>(f.sc, f.prm, f.ps, pass); });
+        [&](const FrameSlot &f) { return pass_work(f, pass, kCtrWorkTransmit); },
+        [&](const FrameSlot &f, const Share &share) {
+            transmit_body<kSphere, kStack, kHet, kAdj>(f.sc, f.prm, f.ps, pass, share);
+        });
 }
 
 
@@ -1828,23 +1911,18 @@ __global__ void k_tonemap(float4 *img, uint32_t n, float gamma, float exposure)
 
 // ------------------------------------------------------------ launchers
 // Persistent pass kernels: the caller's persistent_waves, or by default one
-// wave per 256 paths of the launch (all slots), within [1024, kMaxPersistentWaves] (the
-// traversal spill area holds kSpillThreads threads): large chunks fill 256
-// CUs several times over, and small frames launch fewer waves, which drain
-// sooner (256x256 at 4 spp: 7.8 ms with 1024 waves against 9.9 ms with one
-// path per lane); never more waves than the items need.  Every pass kernel
-// fetches work dynamically or strides over the grid, so the count changes
-// timing only.
+// wave per kTravGrain paths of the launch (all slots), at most
+// kMaxPersistentWaves (the traversal spill area holds kSpillThreads threads);
+// launch_persistent then holds each kernel to the waves the GPU has room for.
+// Waves a queue has no share for leave at once (for_slots).  Every pass kernel
+// deals its queue over the grid it gets, so the count changes timing only.
 uint32_t persistent_waves(uint64_t paths, uint32_t requested, uint32_t spill_threads)
 {
     static_assert(kMaxPersistentWaves * kBlock == kSpillThreads, "one spill row per lane");
-    const uint64_t waves = (paths + kBlock - 1) / kBlock;
     const uint32_t most = spill_threads / kBlock;  // one spill row per lane
-    uint64_t cap = (paths + 255u) / 256u;
-    cap = cap < 1024u ? 1024u : cap;
-    if (requested) cap = requested;
-    cap = cap < most ? cap : most;
-    return (uint32_t)(waves < cap ? (waves ? waves : 1) : cap);
+    const uint64_t waves = (paths + kTravGrain - 1) / kTravGrain;
+    const uint64_t cap = std::min<uint64_t>(requested ? requested : most, most);
+    return (uint32_t)std::max<uint64_t>(std::min(waves, cap), 1);
 }
 
 // ------------------------------------------------------------ multi-frame launchers
