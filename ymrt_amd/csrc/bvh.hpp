@@ -257,8 +257,9 @@ inline uint32_t collapse_wide(const std::vector<BinNode> &bin, std::vector<WNode
                     w.hi_y[k] = b.hi[1];
                     w.hi_z[k] = b.hi[2];
                 } else {
-                    w.lo_x[k] = w.lo_y[k] = w.lo_z[k] = 1.0f;
-                    w.hi_x[k] = w.hi_y[k] = w.hi_z[k] = -1.0f;
+                    // inverted without bound: missed by every ray
+                    w.lo_x[k] = w.lo_y[k] = w.lo_z[k] = INFINITY;
+                    w.hi_x[k] = w.hi_y[k] = w.hi_z[k] = -INFINITY;
                     w.child[k] = kSentinel;
                 }
             }

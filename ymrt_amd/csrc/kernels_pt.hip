@@ -607,10 +607,8 @@ __device__ __forceinline__ void extend_body(const DevScene &sc, const PtParams &
             q.last_inst = last.x;
             q.last_tri = last.y;
             tv.hit.back = 0;
-            tv.hit.inst = kEmpty;
             tv.hit.tri = 0;
             tv.hit.b0 = tv.hit.b1 = tv.hit.b2 = 0.0f;
-            tv.nb_count = 0;
             r = tv.init(sc, q);
         }
         const uint32_t want = rr.want();
@@ -623,6 +621,7 @@ __device__ __forceinline__ void extend_body(const DevScene &sc, const PtParams &
             if (r == kTravOverflow) atomicOr(prm.error, 1u);
             const bool hit = r == kTravHit;
             r = kLaneIdle;
+            if (hit) tv.resolve_backs(sc, ls);
             uint32_t info = gload(ps.info + p);
             if (info & kInfoPendingBunch) {
                 // the boundary bunch of the previous vertex reads that
@@ -1646,7 +1645,7 @@ __device__ __forceinline__ void shadow_body(const DevScene &sc, const PtParams &
 
 
 template <bool kMedia, bool kSphere, int kStack, bool kAdj = false>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_shadow_m(const FrameSlot *__restrict__ fs, uint32_t nfs, uint32_t pass)
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kAdj ? 4 : 5))) void k_shadow_m(const FrameSlot *__restrict__ fs, uint32_t nfs, uint32_t pass)
 {
     for_slots<kTravGrain, kBlock * kSub>(
         fs, nfs, [&](const FrameSlot &f) { return pass_counter(f, pass, kCtrShadow); },

@@ -53,10 +53,6 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace(DevScene sc, const float4
                     q.tmax = r1.w;
                     q.last_inst = kEmpty;
                     q.last_tri = kEmpty;
-                    tv.hit.back = 0;
-                    tv.hit.inst = kEmpty;
-                    tv.hit.tri = kEmpty;
-                    tv.nb_count = 0;
                     cnt = TraceCounters{0, 0};
                     r = tv.init(sc, q);
                 }
@@ -75,6 +71,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace(DevScene sc, const float4
             if (kAny) {
                 occluded[i] = hit ? 1u : 0u;
             } else {
+                if (hit) tv.resolve_backs(sc, ls);
                 hits[i] = hit ? make_uint4(__float_as_uint(tv.hit.t), tv.hit.tri, tv.hit.inst, (uint32_t)tv.hit.back)
                               : make_uint4(__float_as_uint(kTMax), kEmpty, kEmpty, 0u);
             }
