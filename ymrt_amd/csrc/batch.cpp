@@ -234,16 +234,15 @@ int render_batch(ymrt_context *ctx, const ymrt_batch_item *items, uint32_t n, ui
             prm.noise = reinterpret_cast<float4 *>(it.noise_rgba);
             const bool media = rs.enable_volume_scattering && sc->dev.volume_count > 0;
             prm.media = media ? 1u : 0u;
-            // the slot's range of the shared path state (per-path arrays and
-            // queues by offset; arrays of several entries per path keep the
-            // round's capacity as their stride)
+            // the slot's range of the shared path state (per-path records and
+            // queues by offset; arrays with an entry per path and index keep
+            // the round's capacity as their stride)
             PathState ps = rb.ps;
-            auto sh = [&](auto *&p) { p += off; };
-            sh(ps.ray_o), sh(ps.ray_d), sh(ps.last), sh(ps.beta), sh(ps.L), sh(ps.smp), sh(ps.info), sh(ps.xhdr);
-            sh(ps.xrec), sh(ps.hit_a), sh(ps.hit_b), sh(ps.nb), sh(ps.sh_o), sh(ps.sh_d), sh(ps.sh_f), sh(ps.sh_li);
-            sh(ps.sh_tr), sh(ps.sh_c), sh(ps.sh_flags), sh(ps.out), sh(ps.queue[0]), sh(ps.queue[1]), sh(ps.q_hit);
-            sh(ps.q_hit_vol), sh(ps.q_hit_diffuse), sh(ps.q_hit_metal), sh(ps.q_medium), sh(ps.q_shadow);
-            sh(ps.q_transmit), sh(ps.flag), sh(ps.first_hit);
+            auto sh = [&](auto *&p, size_t per_path = 1) { p += off * per_path; };
+            sh(ps.ray, 2), sh(ps.bs, 2), sh(ps.L), sh(ps.xhdr), sh(ps.xrec), sh(ps.hit, 2), sh(ps.nb);
+            sh(ps.sh, kShadowSlots * 4), sh(ps.sh_tr), sh(ps.sh_c), sh(ps.sh_flags), sh(ps.out), sh(ps.queue[0]);
+            sh(ps.queue[1]), sh(ps.q_hit), sh(ps.q_hit_vol), sh(ps.q_hit_diffuse), sh(ps.q_hit_metal);
+            sh(ps.q_medium), sh(ps.q_shadow), sh(ps.q_transmit), sh(ps.flag), sh(ps.first_hit);
             ps.ccount = rb.ps.ccount + (size_t)s * 4 * ccount_stride;
             f.ps = ps;
             off += c.paths;

@@ -53,22 +53,14 @@ inline int layout_buffers(RenderBuffers &rb, size_t n, uint32_t spill_threads, G
 {
     PathState &ps = rb.ps;
     int rc = 0;
-    rc |= get(ps.ray_o, n);
-    rc |= get(ps.ray_d, n);
-    rc |= get(ps.last, n);
-    rc |= get(ps.beta, n);
+    rc |= get(ps.ray, n * 2);
+    rc |= get(ps.bs, n * 2);
     rc |= get(ps.L, n);
-    rc |= get(ps.smp, n);
-    rc |= get(ps.info, n);
     rc |= get(ps.xhdr, n);
     rc |= get(ps.xrec, n * kMaxBoundaryRecord);
-    rc |= get(ps.hit_a, n);
-    rc |= get(ps.hit_b, n);
+    rc |= get(ps.hit, n * 2);
     rc |= get(ps.nb, n * 4);
-    rc |= get(ps.sh_o, n * kShadowSlots);
-    rc |= get(ps.sh_d, n * kShadowSlots);
-    rc |= get(ps.sh_f, n * kShadowSlots);
-    rc |= get(ps.sh_li, n * kShadowSlots);
+    rc |= get(ps.sh, n * kShadowSlots * 4);
     rc |= get(ps.sh_tr, n * kShadowSlots);
     rc |= get(ps.sh_c, n);
     rc |= get(ps.sh_flags, n);

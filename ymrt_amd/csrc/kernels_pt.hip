@@ -416,14 +416,22 @@ __device__ __forceinline__ void store_transfer(const PathState &ps, uint32_t p, 
             ps.xrec[(size_t)i * cap + p] = make_uint4(t.rec[i].prim, __float_as_uint(t.rec[i].ior),
                                                       t.rec[i].priority, (uint32_t)t.rec[i].vol);
 }
-__device__ __forceinline__ NearbyList load_nearby(const PathState &ps, uint32_t p, uint32_t cap, uint32_t hflags)
+// hit flags
+constexpr uint32_t kHitBack = 1u;
+constexpr uint32_t kHitVolume = 2u;
+
+// The nearby list of the path's hit record ha.  A list of one is the hit
+// itself (the instance with the closest hit is always on it) and is not kept
+// apart.
+__device__ __forceinline__ NearbyList load_nearby(const PathState &ps, uint32_t p, uint32_t cap, uint4 ha)
 {
     NearbyList nb;
-    nb.n = (int)((hflags >> 4) & 0xFu);
+    nb.n = (int)((ha.w >> 4) & 0xFu);
 #pragma unroll
     for (int i = 0; i < kNearbyMax; ++i) {
         uint2 e = make_uint2(0u, 0u);
-        if (i < nb.n) e = ps.nb[(size_t)i * cap + p];
+        if (i == 0) e = make_uint2(ha.y | ((ha.w & kHitBack) << 31), ha.x);
+        if (i < nb.n && nb.n > 1) e = ps.nb[(size_t)i * cap + p];
         nb.prim[i] = e.x & 0x7FFFFFFFu;
         nb.back[i] = (int)(e.x >> 31);
         nb.t[i] = __uint_as_float(e.y);
@@ -432,7 +440,7 @@ __device__ __forceinline__ NearbyList load_nearby(const PathState &ps, uint32_t 
 }
 __device__ __forceinline__ Sampler load_sampler(const PathState &ps, uint32_t p)
 {
-    const uint4 s = ps.smp[p];
+    const uint4 s = *ps.smp(p);
     Sampler r;
     r.index = (uint64_t)s.x | ((uint64_t)s.y << 32);
     r.dim = s.z;
@@ -441,7 +449,7 @@ __device__ __forceinline__ Sampler load_sampler(const PathState &ps, uint32_t p)
 }
 __device__ __forceinline__ void store_sampler(const PathState &ps, uint32_t p, const Sampler &s)
 {
-    ps.smp[p] = make_uint4((uint32_t)s.index, (uint32_t)(s.index >> 32), s.dim, s.frame_type);
+    *ps.smp(p) = make_uint4((uint32_t)s.index, (uint32_t)(s.index >> 32), s.dim, s.frame_type);
 }
 
 // info word
@@ -455,10 +463,6 @@ __device__ __forceinline__ uint32_t shade_flag(uint32_t cls)
 {
     return cls == kMatDiffuse ? kFlagDiffuse : cls == kMatMetal ? kFlagMetal : kFlagHit;
 }
-
-// hit flags
-constexpr uint32_t kHitBack = 1u;
-constexpr uint32_t kHitVolume = 2u;
 
 // shadow flags: bits 0-3 shadow ray k recorded (slots 0-1 shape light,
 // 2-3 distant light), 4-7 ray k crosses the surface, 8-11 ray k reached the
@@ -535,13 +539,11 @@ __device__ __forceinline__ void raygen_body(const DevScene &sc, const PtParams &
                 const float height = 2.0f * cam.tan_half_fov;
                 const float width = height * cam.aspect;
                 const f3 dir = normalize(-cam.w + ((nx - 0.5f) * width) * cam.u + ((ny - 0.5f) * height) * cam.v);
-                ps.ray_o[p] = f4(cam.position, 0.0f);
-                ps.ray_d[p] = f4(dir, 0.0f);
-                ps.last[p] = make_uint2(kEmpty, kEmpty);
-                ps.beta[p] = make_float4(1.0f, 1.0f, 1.0f, 0.0f);
+                *ps.ray_o(p) = f4(cam.position, __uint_as_float(kEmpty));
+                *ps.ray_d(p) = f4(dir, __uint_as_float(kEmpty));
+                *ps.beta(p) = make_float4(1.0f, 1.0f, 1.0f, __uint_as_float(1u | kInfoNeverScatter));
                 ps.L[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                 store_sampler(ps, p, smp);
-                ps.info[p] = 1u | kInfoNeverScatter;
                 Transfer t;
                 t.count = cam.record_count;
                 t.max_idx = cam.max_idx;
@@ -597,15 +599,14 @@ __device__ __forceinline__ void extend_body(const DevScene &sc, const PtParams &
         uint32_t item = 0;
         if (rr.more && rr.refill(r == kLaneIdle, item)) {
             p = gload(qin + item);
-            const float4 o4 = gload(ps.ray_o + p), d4 = gload(ps.ray_d + p);
-            const uint2 last = gload(ps.last + p);
+            const float4 o4 = gload(ps.ray_o(p)), d4 = gload(ps.ray_d(p));
             Query q;
             q.o = xyz(o4);
             q.d = xyz(d4);
             q.tmin = kTMin;
             q.tmax = kTMax;
-            q.last_inst = last.x;
-            q.last_tri = last.y;
+            q.last_inst = __float_as_uint(o4.w);
+            q.last_tri = __float_as_uint(d4.w);
             tv.hit.back = 0;
             tv.hit.tri = 0;
             tv.hit.b0 = tv.hit.b1 = tv.hit.b2 = 0.0f;
@@ -622,16 +623,16 @@ __device__ __forceinline__ void extend_body(const DevScene &sc, const PtParams &
             const bool hit = r == kTravHit;
             r = kLaneIdle;
             if (hit) tv.resolve_backs(sc, ls);
-            uint32_t info = gload(ps.info + p);
+            uint32_t info = gload(ps.info(p));
             if (info & kInfoPendingBunch) {
                 // the boundary bunch of the previous vertex reads that
                 // vertex's nearby list, which the writes below replace
                 Transfer t = load_transfer(ps, p, prm.cap);
-                const NearbyList nb = load_nearby(ps, p, prm.cap, ps.hit_a[p].w);
+                const NearbyList nb = load_nearby(ps, p, prm.cap, *ps.hit_a(p));
                 boundary_bunch(sc, t, nb);
                 store_transfer(ps, p, prm.cap, t);
                 info &= ~kInfoPendingBunch;
-                ps.info[p] = info;
+                *ps.info(p) = info;
             }
             rays += 1;
             cam_rays += (info_depth(info) == 1 && (info & kInfoNeverScatter)) ? 1u : 0u;
@@ -641,7 +642,7 @@ __device__ __forceinline__ void extend_body(const DevScene &sc, const PtParams &
             if (!hit && !in_medium) {
                 f3 Lv = xyz(gload(ps.L + p));
                 if (rs.enable_env_light)
-                    Lv = Lv + light_clamp(rs, xyz(gload(ps.beta + p)) * background(tv.q.d), info_depth(info));
+                    Lv = Lv + light_clamp(rs, xyz(gload(ps.beta(p))) * background(tv.q.d), info_depth(info));
                 gstore(ps.out + p, f4(Lv, 0.0f));
             } else {
                 // a path in a medium may have no surface hit (h.inst empty);
@@ -649,12 +650,10 @@ __device__ __forceinline__ void extend_body(const DevScene &sc, const PtParams &
                 const uint32_t mat = hit ? gload(&sc.instances[h.inst].material) : kEmpty;
                 gstore(ps.flag + p, (pass << kFlagBits) | (in_medium ? kFlagMedium : shade_flag(gload(sc.mat_class + mat))));
                 uint32_t flags = h.back ? kHitBack : 0u;
-                bool listed = false;
-                const int nbc = tv.nb_count;
+                int nbc = hit ? 1 : 0;  // without the list the hit is its own nearby hit
                 if constexpr (kNearby) {
-                    if (hit) {
-                        listed = true;
-                        flags |= (uint32_t)nbc << 4;
+                    if (hit) nbc = tv.nb_count;
+                    if (nbc > 1)
                         static_for<0, kNearbyCap>([&](auto K) {
                             if (K() < nbc)
                                 gstore(ps.nb + (size_t)K() * prm.cap + p,
@@ -662,15 +661,10 @@ __device__ __forceinline__ void extend_body(const DevScene &sc, const PtParams &
                                                       ((uint32_t)(nbb[K() * kBlock + lane_id()] != 0) << 31),
                                                   __float_as_uint(nbt[K() * kBlock + lane_id()])));
                         });
-                    }
                 }
-                if (!listed && hit) {
-                    // without the list the closest instance is its own nearby hit
-                    flags |= 1u << 4;
-                    gstore(ps.nb + p, make_uint2(h.inst | ((uint32_t)(h.back != 0) << 31), __float_as_uint(h.t)));
-                }
-                gstore(ps.hit_a + p, make_uint4(__float_as_uint(hit ? h.t : kTMax), hit ? h.inst : kEmpty, h.tri, flags));
-                gstore(ps.hit_b + p, make_float4(h.b0, h.b1, h.b2, 0.0f));
+                flags |= (uint32_t)nbc << 4;
+                gstore(ps.hit_a(p), make_uint4(__float_as_uint(hit ? h.t : kTMax), hit ? h.inst : kEmpty, h.tri, flags));
+                gstore(ps.hit_b(p), make_float4(h.b0, h.b1, h.b2, 0.0f));
             }
         }
         if (!rr.more && __ballot(r != kLaneIdle) == 0) break;
@@ -894,10 +888,11 @@ __device__ __forceinline__ void medium_body(const DevScene &sc, const PtParams &
     run_items<0, kMediumSub>(share, cnt + kCtrWorkMedium, n, nullptr, nullptr, [&](uint32_t i, uint32_t &p, bool(&)[1]) {
         {
             p = ps.q_medium[i];
-            const uint4 ha = ps.hit_a[p];
+            const uint4 ha = *ps.hit_a(p);
             const bool hit = ha.y != kEmpty;
-            const f3 o = xyz(ps.ray_o[p]), d = xyz(ps.ray_d[p]);
-            f3 beta = xyz(ps.beta[p]);
+            const f3 o = xyz(*ps.ray_o(p)), d = xyz(*ps.ray_d(p));
+            const float4 bi = *ps.beta(p);
+            f3 beta = xyz(bi);
             bool vol_hit = false;
             float dist = 0.0f;
             const Transfer t = load_transfer(ps, p, prm.cap);
@@ -934,19 +929,19 @@ __device__ __forceinline__ void medium_body(const DevScene &sc, const PtParams &
                     vol_hit = sample_homogeneous(sc, nv, vi, tmax, trw, dist, smp);
                 }
                 beta = beta * trw;
-                ps.beta[p] = f4(beta, 0.0f);
+                *ps.beta(p) = f4(beta, bi.w);
                 store_sampler(ps, p, smp);
             }
             if (vol_hit) {
                 ps.flag[p] = (pass << kFlagBits) | kFlagVolume;
                 const f3 vpos = o + d * dist;
-                ps.hit_a[p] = make_uint4(ha.x, ha.y, ha.z, ha.w | kHitVolume);
-                ps.hit_b[p] = make_float4(vpos.x, vpos.y, vpos.z, 0.0f);
+                *ps.hit_a(p) = make_uint4(ha.x, ha.y, ha.z, ha.w | kHitVolume);
+                *ps.hit_b(p) = make_float4(vpos.x, vpos.y, vpos.z, 0.0f);
             } else if (hit) {
                 ps.flag[p] = (pass << kFlagBits) | shade_flag(sc.mat_class[sc.instances[ha.y].material]);
             } else {
                 f3 Lv = xyz(ps.L[p]);
-                if (rs.enable_env_light) Lv = Lv + light_clamp(rs, beta * background(d), info_depth(ps.info[p]));
+                if (rs.enable_env_light) Lv = Lv + light_clamp(rs, beta * background(d), info_depth(__float_as_uint(bi.w)));
                 ps.out[p] = f4(Lv, 0.0f);
             }
         }
@@ -1004,17 +999,17 @@ __device__ __forceinline__ void adj_texels(const DevScene &sc, const AdjParams &
 // with no spawn offset.
 struct ShadowEmit {
     const PathState &ps;
-    uint32_t cap, p;
+    uint32_t p;
     uint32_t flags;
     // g: the adjoint replay's d ln f / d r of the ray's BSDF value (0 otherwise)
     __device__ __forceinline__ void emit(int k, f3 orig, f3 dir, float tmax, bool transmit, f3 f, f3 li, float mis,
                                          float g = 0.0f)
     {
-        const size_t o = (size_t)k * cap + p;
-        ps.sh_o[o] = f4(orig, tmax);
-        ps.sh_d[o] = f4(normalize(dir), 0.0f);
-        ps.sh_f[o] = f4(f, mis);
-        ps.sh_li[o] = f4(li, g);
+        float4 *r = ps.shadow(k, p);
+        r[0] = f4(orig, tmax);
+        r[1] = f4(normalize(dir), 0.0f);
+        r[2] = f4(f, mis);
+        r[3] = f4(li, g);
         flags |= (1u << k) | (transmit ? (kShTransmit0 << k) : 0u);
     }
 };
@@ -1069,18 +1064,19 @@ __device__ __forceinline__ void shade_body(const DevScene &sc, const PtParams &p
                  [&](uint32_t i, uint32_t &p, bool(&out)[2]) {
         {
             p = q[i];
-            uint32_t info = ps.info[p];
+            const float4 bi = *ps.beta(p);
+            uint32_t info = __float_as_uint(bi.w);
             int depth = info_depth(info);
             bool never_scatter = (info & kInfoNeverScatter) != 0;
             const uint32_t vertex = info_vertex(info) + 1;
-            const uint4 ha = ps.hit_a[p];
-            const float4 hb = ps.hit_b[p];
-            const f3 ray_d = xyz(ps.ray_d[p]);
-            f3 beta = xyz(ps.beta[p]);
-            f3 L = xyz(ps.L[p]);
+            const uint4 ha = *ps.hit_a(p);
+            const float4 hb = *ps.hit_b(p);
+            const f3 ray_d = xyz(*ps.ray_d(p));
+            f3 beta = xyz(bi);
             Sampler smp = load_sampler(ps, p);
-            ShadowEmit so{ps, cap, p, (uint32_t)depth << kShDepthShift};
+            ShadowEmit so{ps, p, (uint32_t)depth << kShDepthShift};
             bool alive = false;       // a next extension ray
+            f3 emitted = s3(0.0f);    // radiance of a light the path ends on
             const f3 sh_beta = beta;
             float sel_pdf = 0.0f;
             f3 next_o = s3(0.0f), next_d = s3(0.0f);
@@ -1234,9 +1230,9 @@ __device__ __forceinline__ void shade_body(const DevScene &sc, const PtParams &p
                     next_lt = tri;
                 } else if (mtype == YMRT_MATERIAL_LIGHT) {
                     if (never_scatter)
-                        L = L + light_clamp(rs, beta * f3{m.light_color[0], m.light_color[1], m.light_color[2]} *
-                                                    m.intensity,
-                                            depth);
+                        emitted = light_clamp(rs, beta * f3{m.light_color[0], m.light_color[1], m.light_color[2]} *
+                                                      m.intensity,
+                                              depth);
                 } else {
                     f3 sn, dpdu, dpdv;
                     f2 uv;
@@ -1307,7 +1303,7 @@ __device__ __forceinline__ void shade_body(const DevScene &sc, const PtParams &p
                         const bool tex_on = A.tex != kEmpty && m.diffuse_albedo_tex == A.tex;
                         rough_entry = A.rough_slot[in.material];
                         if (as >= 0 || tex_on || rough_entry >= 0)
-                            adj_dl = adj_pixel(prm, p) * (xyz(ps.out[p]) - L);
+                            adj_dl = adj_pixel(prm, p) * (xyz(ps.out[p]) - xyz(ps.L[p]));
                         if (as >= 0) {
 #pragma unroll
                             for (int c = 0; c < 3; ++c) {
@@ -1456,25 +1452,28 @@ __device__ __forceinline__ void shade_body(const DevScene &sc, const PtParams &p
             // ---------------------------------------------- write back
             const bool nee = (so.flags & kShActiveMask) != 0;
             store_sampler(ps, p, smp);
-            ps.L[p] = f4(L, 0.0f);
             if (nee) {
                 out[0] = true;
                 if (!alive) so.flags |= kShTerminate;
                 ps.sh_flags[p] = so.flags;
                 ps.sh_c[p] = f4(sh_beta, sel_pdf);
             } else if (!alive) {
-                ps.out[p] = f4(L, 0.0f);
-            }
-            if (alive) {
-                out[1] = true;
-                ps.ray_o[p] = f4(next_o, 0.0f);
-                ps.ray_d[p] = f4(next_d, 0.0f);
-                ps.last[p] = make_uint2(next_li, next_lt);
-                ps.beta[p] = f4(beta, 0.0f);
+                // the path's radiance changes here only where it ends on a
+                // light; elsewhere it stays in HBM (adding 0 to -0 gives the
+                // same output as the reference's sum: a path's radiance
+                // starts at +0)
+                ps.out[p] = f4(xyz(ps.L[p]) + emitted, 0.0f);
             }
             info = (uint32_t)depth | (never_scatter ? kInfoNeverScatter : 0u) | (pending ? kInfoPendingBunch : 0u) |
                    (vertex << 16);
-            ps.info[p] = info;
+            if (alive) {
+                out[1] = true;
+                *ps.ray_o(p) = f4(next_o, __uint_as_float(next_li));
+                *ps.ray_d(p) = f4(next_d, __uint_as_float(next_lt));
+                *ps.beta(p) = f4(beta, __uint_as_float(info));
+            } else if (nee) {
+                *ps.info(p) = info;  // the transmittance stage's random numbers are keyed by the vertex
+            }
         }
     });
     sums.end();
@@ -1520,10 +1519,9 @@ __device__ __forceinline__ void shadow_finish(const PtParams &prm, const PathSta
         rc[K()] = s3(0.0f);
         rg[K()] = 0.0f;
         if ((fl & (1u << K())) && (fl & (kShClear0 << K()))) {
-            const size_t o = (size_t)K() * cap + p;
-            const float4 f4v = ps.sh_f[o];
-            const float4 li4 = ps.sh_li[o];
-            const f3 tr = with_tr ? xyz(ps.sh_tr[o]) : s3(1.0f);
+            const float4 f4v = ps.shadow(K(), p)[2];
+            const float4 li4 = ps.shadow(K(), p)[3];
+            const f3 tr = with_tr ? xyz(ps.sh_tr[(size_t)K() * cap + p]) : s3(1.0f);
             const f3 c = ((f4v.w * tr) * xyz(f4v)) * xyz(li4);
             if (K() < 2) shape = shape + c;
             else dist = dist + c;
@@ -1576,7 +1574,6 @@ __device__ __forceinline__ void shadow_body(const DevScene &sc, const PtParams &
     AdjSums<kAdj> sums{adj_lds, &prm.adj};
     sums.begin();
     uint32_t *cnt = prm.counters + pass * kCtrStride;
-    const uint32_t cap = prm.cap;
     LaneScratch<kBlock, kStackWindow, true> ls{stack, nullptr, nullptr, nullptr, (int)lane_id(), ps.spill,
                                                ps.spill_threads, blockIdx.x * kBlock + threadIdx.x, pre_park};
     uint32_t nsh = 0;
@@ -1589,8 +1586,8 @@ __device__ __forceinline__ void shadow_body(const DevScene &sc, const PtParams &
     int k = 0;
     int r = kLaneIdle;
     auto start_ray = [&]() {
-        const float4 o4 = gload(ps.sh_o + (size_t)k * cap + p);
-        const float4 d4 = gload(ps.sh_d + (size_t)k * cap + p);
+        const float4 o4 = gload(ps.shadow(k, p));
+        const float4 d4 = gload(ps.shadow(k, p) + 1);
         Query q;
         q.o = xyz(o4);
         q.d = xyz(d4);
@@ -1689,8 +1686,8 @@ __device__ __forceinline__ void transmit_body(const DevScene &sc, const PtParams
             const uint32_t p = ps.q_transmit[i];
             slot = p;
             const uint32_t fl = ps.sh_flags[p];
-            const uint32_t info = ps.info[p];
-            const uint4 ha = ps.hit_a[p];
+            const uint32_t info = *ps.info(p);
+            const uint4 ha = *ps.hit_a(p);
             HashRng rng;
             {
                 // 64-bit like k_raygen: a frame may hold more than 2^32 path slots
@@ -1713,13 +1710,13 @@ __device__ __forceinline__ void transmit_body(const DevScene &sc, const PtParams
                 const int k = (j + 2) & 3;
                 if (!(fl & (1u << k)) || !(fl & (kShClear0 << k))) continue;
                 auto walk = [&](auto &&ev) -> f3 {
-                    const float4 o4 = ps.sh_o[(size_t)k * cap + p];
-                    const float4 d4 = ps.sh_d[(size_t)k * cap + p];
+                    const float4 o4 = ps.shadow(k, p)[0];
+                    const float4 d4 = ps.shadow(k, p)[1];
                     f3 tr = s3(1.0f);
                     // the vertex's records and nearby list are reloaded per ray
                     // rather than held across the loop (fewer live registers)
                     Transfer t = load_transfer(ps, p, cap);
-                    if (fl & (kShTransmit0 << k)) boundary_bunch(sc, t, load_nearby(ps, p, cap, ha.w));
+                    if (fl & (kShTransmit0 << k)) boundary_bunch(sc, t, load_nearby(ps, p, cap, ha));
                     const bool volv = (fl & kShVolume) != 0;
                     Query tq;
                     tq.o = xyz(o4);
@@ -1775,9 +1772,8 @@ __device__ __forceinline__ void transmit_body(const DevScene &sc, const PtParams
                 if constexpr (kAdj && kHet > 0) {
                     if (prm.adj.vol != kEmpty) {
                         // this ray's deposit, as shadow_finish sums it
-                        const size_t o = (size_t)k * cap + p;
-                        const float4 f4v = ps.sh_f[o];
-                        const float4 li4 = ps.sh_li[o];
+                        const float4 f4v = ps.shadow(k, p)[2];
+                        const float4 li4 = ps.shadow(k, p)[3];
                         const float4 c4 = ps.sh_c[p];
                         const f3 c = ((f4v.w * tr) * xyz(f4v)) * xyz(li4);
                         const float scale = k >= 2 ? (float)sc.distant_count
