@@ -214,16 +214,21 @@ private:
 // Collapses a binary tree into WNodes appended to `out`.  Leaf prims are the
 // ranges [first, first+count) of the builder's prim order, offset by
 // prim_base.  Returns the root code (node index, or a leaf code when the
-// whole tree is one leaf) and the wide depth in *depth.
+// whole tree is one leaf) and the wide depth in *depth.  leaves: the codes of
+// single-primitive leaves by BinNode::first, in place of leaf codes (the
+// top-level trees).
 inline uint32_t collapse_wide(const std::vector<BinNode> &bin, std::vector<WNode> &out, uint32_t prim_base,
-                              uint32_t *depth)
+                              uint32_t *depth, const uint32_t *leaves = nullptr)
 {
     *depth = 0;
     if (bin.empty()) return kSentinel;
-    if (bin[0].left < 0) return leaf_code(prim_base + bin[0].first, bin[0].count);
     struct Rec {
+        static uint32_t leaf(const BinNode &n, uint32_t base, const uint32_t *leaves)
+        {
+            return leaves ? leaves[n.first] : leaf_code(base + n.first, n.count);
+        }
         static uint32_t go(const std::vector<BinNode> &bin, std::vector<WNode> &out, uint32_t base, int32_t bi,
-                           uint32_t level, uint32_t *depth)
+                           uint32_t level, uint32_t *depth, const uint32_t *leaves)
         {
             *depth = std::max(*depth, level + 1);
             int32_t kids[4] = {bin[bi].left, bin[bi].right, -1, -1};
@@ -266,16 +271,17 @@ inline uint32_t collapse_wide(const std::vector<BinNode> &bin, std::vector<WNode
             for (int k = 0; k < nk; ++k) {
                 const BinNode &c = bin[kids[k]];
                 if (c.left < 0) {
-                    w.child[k] = leaf_code(base + c.first, c.count);
+                    w.child[k] = leaf(c, base, leaves);
                 } else {
-                    w.child[k] = go(bin, out, base, kids[k], level + 1, depth);
+                    w.child[k] = go(bin, out, base, kids[k], level + 1, depth, leaves);
                 }
             }
             out[me] = w;
             return me;
         }
     };
-    return Rec::go(bin, out, prim_base, 0, 0, depth);
+    if (bin[0].left < 0) return Rec::leaf(bin[0], prim_base, leaves);
+    return Rec::go(bin, out, prim_base, 0, 0, depth, leaves);
 }
 
 }  // namespace ym

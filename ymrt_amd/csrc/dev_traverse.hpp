@@ -322,8 +322,8 @@ struct TraceCounters {
     } while (0)
 
 // Resumable traversal: init() then step() until it returns something other
-// than kTravContinue.  One step visits one wide node, one top-level leaf
-// (an instance entry or a sphere) or one bottom-level leaf, then pops the
+// than kTravContinue.  One step visits one wide node, one instance leaf (an
+// instance entry or a sphere) or one triangle leaf, then pops the
 // next entry, so a caller can interleave rays (a lane that finishes can
 // start another ray while the rest of its wave traverses).
 // kSphere: the scene has sphere instances (their test is compiled in only
@@ -347,10 +347,14 @@ struct Traversal {
     RayPre pre;
     Hit hit;                  // hit.inst kEmpty: nothing hit so far
     float tbest;
-    uint32_t node, cur_inst;  // cur_inst: the instance being traversed, or kEmpty
+    uint32_t node, cur_inst;  // cur_inst: the instance the ray has entered, or kEmpty
     int sp, nb_count;
-    // the current instance's nearest crossing, hit or not, and the side code
-    // of its last tested one
+    // nearby list: the instance whose crossings are being collected, entered
+    // or linked (kEmpty: none), its nearest crossing, hit or not, and the side
+    // code of its last tested one.  A linked mesh's subtree is traversed in
+    // one piece like an entered one, so its crossings end where another
+    // instance's begin.
+    uint32_t near_inst;
     float ex_t;
     int ex_code;
     float tub, tlb;
@@ -373,6 +377,7 @@ struct Traversal {
         pre = make_pre(q.o, q.d);
         tbest = q.tmax;
         cur_inst = kEmpty;
+        near_inst = kEmpty;
         ex_t = INFINITY;
         ex_code = 0;
         tub = 0.0f;
@@ -382,12 +387,15 @@ struct Traversal {
         return kTravContinue;
     }
 
-    // nearby-list update when the traversal leaves an instance (TraceRay's
-    // per-instance block, src/ShadingUtilities.cuh:357-393)
+    // Starts collecting the crossings of instance `inst` (kEmpty: of none)
+    // and settles those of the one before: the nearby-list update at the end
+    // of an instance (TraceRay's per-instance block,
+    // src/ShadingUtilities.cuh:357-393).
     template <typename LS>
-    YM_HD void nearby_exit(LS &ls)
+    YM_HD void nearby_open(LS &ls, uint32_t inst)
     {
-        if (hit.inst == cur_inst && cur_inst != kEmpty) {
+        if (near_inst == kEmpty) {
+        } else if (hit.inst == near_inst) {
             tub = next_float_up(next_float_up(tbest));
             tlb = next_float_down(next_float_down(tbest));
             int w = 0;
@@ -402,19 +410,21 @@ struct Traversal {
             }
             nb_count = w;
             if (nb_count < kNearbyCap) {
-                ls.nb_prim[ls.nbi(nb_count)] = cur_inst;
+                ls.nb_prim[ls.nbi(nb_count)] = near_inst;
                 ls.nb_t[ls.nbi(nb_count)] = tbest;
                 ls.nb_back[ls.nbi(nb_count)] = hit_code();
                 ++nb_count;
             }
         } else if (hit.inst != kEmpty && ex_t > tlb && ex_t < tub) {
             if (nb_count < kNearbyCap) {
-                ls.nb_prim[ls.nbi(nb_count)] = cur_inst;
+                ls.nb_prim[ls.nbi(nb_count)] = near_inst;
                 ls.nb_t[ls.nbi(nb_count)] = ex_t;
                 ls.nb_back[ls.nbi(nb_count)] = ex_code;
                 ++nb_count;
             }
         }
+        near_inst = inst;
+        ex_t = INFINITY;
     }
 
     // The sides of the hit and of the nearby list's entries, once the
@@ -422,6 +432,7 @@ struct Traversal {
     template <typename LS>
     YM_HD void resolve_backs(const DevScene &sc, LS &ls)
     {
+        if (kNearby) nearby_open(ls, kEmpty);
         const bool sphere = kSphere && hit.tri == kEmpty;
         if (!sphere) hit.back = tri_hit_back(sc, hit.inst, hit.tri, q.d);
         if (kNearby) {
@@ -444,7 +455,7 @@ struct Traversal {
             pre = ls.unpark_pre(q.o, q.d);
         else
             pre = make_pre(q.o, q.d);
-        if (kNearby) nearby_exit(ls);
+        if (kNearby) nearby_open(ls, kEmpty);
         cur_inst = kEmpty;
     }
 
@@ -565,13 +576,14 @@ struct Traversal {
         }
         if (!(node & kLeafBit)) {
             return visit_node<true>(sc, ls, cnt);
-        } else if (!in_blas()) {
-            // top-level leaf: one instance
+        } else if (leaf_is_instance(node)) {
+            // top-level leaf: an instance to enter
             const uint32_t ii = leaf_first(node);
             const DevInstance in = gload(sc.instances + ii);
             bool take = true;
             if (kMode == kModeSkipBoundary) take = !(in.flags & kInstBoundary);
             if (kMode == kModeBoundaryOnly) take = (in.flags & kInstBoundary) != 0;
+            if (kNearby && take) nearby_open(ls, ii);
             if (kSphere && take && (in.flags & kInstSphere)) {
                 SphereTest st;
                 const bool acc = sphere_test(xf_point(in.w2o, q.o), xf_dir(in.w2o, q.d), in.radius, q.tmin, tbest, st);
@@ -590,11 +602,9 @@ struct Traversal {
                     if (kAny) return kTravHit;
                 }
                 if (kNearby) {
-                    cur_inst = ii;
                     ex_t = st.ex_hit ? st.ex_t : INFINITY;
                     ex_code = sphere_code(st.ex_back);
-                    nearby_exit(ls);
-                    cur_inst = kEmpty;
+                    nearby_open(ls, kEmpty);
                 }
             } else if (take) {
                 if (sp + 1 > kStack) return kTravOverflow;
@@ -602,7 +612,6 @@ struct Traversal {
                 if constexpr (LS::kParkPre) ls.park_pre(pre);
                 pre = make_pre(xf_point(in.w2o, q.o), xf_dir(in.w2o, q.d));
                 cur_inst = ii;
-                ex_t = INFINITY;
                 node = in.blas_root;
                 return kTravContinue;
             }
@@ -612,12 +621,14 @@ struct Traversal {
                 const float4 *tp = sc.tris + 3u * (first + k);
                 const float4 w0 = gload(tp), w1 = gload(tp + 1), w2 = gload(tp + 2);
                 const uint32_t tri = f2u(w0.w);
+                const uint32_t inst = in_blas() ? cur_inst : f2u(w1.w);
+                if (kNearby && inst != near_inst) nearby_open(ls, inst);
                 if (kCount) cnt.tris++;
                 const f3 q0{w0.x, w0.y, w0.z}, q1{w1.x, w1.y, w1.z}, q2{w2.x, w2.y, w2.z};
                 TriHit th;
                 // the triangle the ray left: q.last_* are kEmpty without one,
-                // which neither cur_inst nor a triangle id is
-                const bool left = cur_inst == q.last_inst && tri == q.last_tri;
+                // which neither an instance nor a triangle id is
+                const bool left = inst == q.last_inst && tri == q.last_tri;
                 if (!tri_test(pre, q0, q1, q2, th) || left) continue;
                 if (kNearby && th.t >= q.tmin) {
                     ex_t = gmin(ex_t, th.t);
@@ -626,7 +637,7 @@ struct Traversal {
                 if (th.t < q.tmin || th.t > tbest) continue;
                 tbest = th.t;
                 hit.t = th.t;
-                hit.inst = cur_inst;
+                hit.inst = inst;
                 hit.tri = tri;
                 if (!kAny) {
                     hit.b0 = th.e0 * th.inv;

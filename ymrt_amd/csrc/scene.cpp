@@ -294,6 +294,13 @@ static void light_emission_of(const DevMaterial &m, float le[3])
     for (int c = 0; c < 3; ++c) le[c] = m.light_color[c] * m.intensity;
 }
 
+static bool is_identity(const Affine &m)
+{
+    for (int k = 0; k < 12; ++k)
+        if (!(m.r[k] == (k % 5 == 0 ? 1.0f : 0.0f))) return false;
+    return true;
+}
+
 int build_scene(ymrt_scene *sc, const ymrt_scene_desc *d)
 {
     auto t0 = std::chrono::high_resolution_clock::now();
@@ -306,6 +313,7 @@ int build_scene(ymrt_scene *sc, const ymrt_scene_desc *d)
     HostScene h;
     // ---------------------------------------------------------------- meshes
     std::vector<uint32_t> blas_root(d->mesh_count), shade_base(d->mesh_count), mesh_flags(d->mesh_count, 0);
+    std::vector<uint32_t> tri_bases(d->mesh_count);
     uint32_t max_blas_depth = 0;
     uint64_t total_tris = 0;
     for (uint32_t mi = 0; mi < d->mesh_count; ++mi) {
@@ -363,7 +371,10 @@ int build_scene(ymrt_scene *sc, const ymrt_scene_desc *d)
         }
         uint32_t tri_base = (uint32_t)(h.tris.size() / 3);
         YM_REQUIRE((uint64_t)tri_base + m.triangle_count < (1ull << 28), "too many triangles for leaf encoding");
-        BinaryBuilder bb(prims, 4);
+        tri_bases[mi] = tri_base;
+        constexpr uint32_t kLeafPrims = 4;
+        static_assert(kLeafPrims <= kMaxLeafPrims, "leaf size 8 is the instance code");
+        BinaryBuilder bb(prims, kLeafPrims);
         std::vector<BinNode> bin = bb.build();
         uint32_t depth = 0;
         blas_root[mi] = collapse_wide(bin, h.nodes, tri_base, &depth);
@@ -371,7 +382,7 @@ int build_scene(ymrt_scene *sc, const ymrt_scene_desc *d)
         for (const BuildPrim &bp : prims) {
             const ShadeTri &st = h.shade[shade_base[mi] + bp.id];
             h.tris.push_back(make_float4(st.p[0], st.p[1], st.p[2], u2f(bp.id)));
-            h.tris.push_back(make_float4(st.p[3], st.p[4], st.p[5], 0.0f));
+            h.tris.push_back(make_float4(st.p[3], st.p[4], st.p[5], u2f(kEmpty)));
             h.tris.push_back(make_float4(st.p[6], st.p[7], st.p[8], 0.0f));
         }
     }
@@ -383,7 +394,10 @@ int build_scene(ymrt_scene *sc, const ymrt_scene_desc *d)
     }
     // ------------------------------------------------------------- instances
     std::vector<BuildPrim> iprims;
+    std::vector<uint32_t> top_leaf;  // per instance: its code in the top-level trees
+    std::vector<bool> linked(d->mesh_count, false);
     uint32_t has_boundaries = 0, has_spheres = 0;
+    YM_REQUIRE(d->instance_count < (1u << 28) - 1u, "too many instances for leaf encoding");
     for (uint32_t i = 0; i < d->instance_count; ++i) {
         const ymrt_instance_desc &id = d->instances[i];
         YM_REQUIRE(id.geometry_type == YMRT_GEOMETRY_MESH || id.geometry_type == YMRT_GEOMETRY_SPHERE,
@@ -409,7 +423,13 @@ int build_scene(ymrt_scene *sc, const ymrt_scene_desc *d)
         has_spheres |= sphere ? 1u : 0u;
         total_tris += in.tri_count;
         h.instances.push_back(in);
+        top_leaf.push_back(instance_code(i));
         if (!sphere && in.tri_count == 0) continue;
+        if (!sphere && !linked[id.geometry] && is_identity(in.w2o)) {
+            linked[id.geometry] = true;
+            top_leaf[i] = in.blas_root;
+            for (uint32_t t = 0; t < in.tri_count; ++t) h.tris[3ull * (tri_bases[id.geometry] + t) + 1].w = u2f(i);
+        }
         // world bounds: of the transformed vertices for a mesh (a rotated
         // mesh's transformed object box can be far larger, and every ray
         // through the excess enters the instance for nothing), of the
@@ -460,7 +480,7 @@ int build_scene(ymrt_scene *sc, const ymrt_scene_desc *d)
         for (BinNode &n : bin)
             if (n.left < 0) n.first = sel[n.first].id;
         uint32_t depth = 0;
-        uint32_t root = collapse_wide(bin, h.nodes, 0, &depth);
+        uint32_t root = collapse_wide(bin, h.nodes, 0, &depth, top_leaf.data());
         tlas_depth = std::max(tlas_depth, depth);
         return root;
     };
