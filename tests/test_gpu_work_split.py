@@ -1,5 +1,5 @@
 """How the pass kernels deal their queues over the waves of a launch: shares
-of 16 to 256 items by queue length, the first of them without atomics, and in
+of 64 to 256 items by queue length, the first of them without atomics, and in
 a batch one deal over the queues of all frames.  Whatever the deal, every path
 is handled once: frames are bit-identical to the one that a single wave per
 kernel renders, which takes every share in order."""

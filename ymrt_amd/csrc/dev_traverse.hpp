@@ -303,6 +303,18 @@ struct LaneScratch {
     }
 };
 
+// What the steps of a traversal read, apart from its start and results.  A
+// kernel that reads its scene from device memory copies it first: a step
+// would otherwise reload the pointers, which its own stores might change as
+// far as the compiler can tell, before each of its loads (interior, 64 spp:
+// 792 -> 780 ms).
+struct TravScene {
+    const WNode *nodes;
+    const float4 *tris;
+    const DevInstance *instances;
+    YM_HD explicit TravScene(const DevScene &sc) : nodes(sc.nodes), tris(sc.tris), instances(sc.instances) {}
+};
+
 struct TraceCounters {
     uint32_t nodes, tris;
 };
@@ -486,8 +498,8 @@ struct Traversal {
     // with the deferred sides and the flags taken out, took the closest-hit
     // kernel of the interior at 1080p and 1 spp from 1088 to 890 us per pass,
     // the shadow kernel from 556 to 510, and the 64-spp frame from 950 to 879 ms.
-    template <bool kThrough, typename LS>
-    YM_HD int visit_node(const DevScene &sc, LS &ls, TraceCounters &cnt)
+    template <bool kThrough, typename SC, typename LS>
+    YM_HD int visit_node(const SC &sc, LS &ls, TraceCounters &cnt)
     {
         {
             const char *n = reinterpret_cast<const char *>(sc.nodes + node);
@@ -567,8 +579,8 @@ struct Traversal {
         return pop<kThrough>(ls);
     }
 
-    template <typename LS>
-    YM_HD int step(const DevScene &sc, LS &ls, TraceCounters &cnt)
+    template <typename SC, typename LS>
+    YM_HD int step(const SC &sc, LS &ls, TraceCounters &cnt)
     {
         if (node == kSentinel) {
             leave_instance(ls);
@@ -662,8 +674,8 @@ struct Traversal {
 // which end at their first hit.  Measured best on the interior frame:
 // kInnerFirst 16 with the loop (closest hit), 24 without (shadow rays); 8
 // and 32 were slower for both.
-template <int kInnerFirst, bool kLoop, class TV, class LS>
-__device__ __forceinline__ void wave_step(TV &tv, int &r, const DevScene &sc, LS &ls, TraceCounters &tc)
+template <int kInnerFirst, bool kLoop, class TV, class SC, class LS>
+__device__ __forceinline__ void wave_step(TV &tv, int &r, const SC &sc, LS &ls, TraceCounters &tc)
 {
     if constexpr (kLoop) {
         for (;;) {

@@ -31,6 +31,8 @@ constexpr int kBlock = 64;
 
 // ------------------------------------------------------------ wave helpers
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
+// a value that all lanes of the wave hold, kept in a scalar register
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // Items a wave takes per work fetch: up to kSub sub-batches of 64.  Every
 // global counter here is touched by all waves of the grid, and device-scope
@@ -42,9 +44,6 @@ __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 // best for the others.  Short queues are dealt in smaller shares (Share).
 constexpr int kSub = 4;
 constexpr int kRaygenSub = 32, kMediumSub = 8;
-// Smallest share of the traversal kernels, whose lanes refill on their own:
-// with fewer rays than lanes a wave holds kTravGrain of them.
-constexpr int kTravGrain = 16;
 
 // A wave's part of one slot's queue.  The first dealt() items of the queue
 // are dealt without atomics: the slot's home waves take grain() items each,
@@ -139,7 +138,8 @@ struct RefillRange {
     uint32_t cur, end;
     bool more;  // the range or the work counter may hold items
     __device__ __forceinline__ RefillRange(const Share &s, uint32_t *w, uint32_t count)
-        : share(s), work(w), n(count), cur(s.first), end(s.first_end), more(s.first < s.first_end || s.dealt() < count)
+        : share(s), work(w), n(uniform(count)), cur(uniform(s.first)), end(uniform(s.first_end)),
+          more(cur < end || s.dealt() < n)
     {
     }
     __device__ __forceinline__ bool refill(bool idle_lane, uint32_t &item)
@@ -160,7 +160,7 @@ struct RefillRange {
                     took = true;
                 }
             }
-            cur += take;
+            cur = uniform(cur + take);
             idle = __ballot(idle_lane && !took);
         }
         // a queue dealt in full has nothing to fetch
@@ -320,14 +320,17 @@ __device__ __forceinline__ uint32_t *pass_work(const FrameSlot &f, uint32_t pass
 //   * kMaxGrain when every wave of the grid gets that many: long queues, whose
 //     fetch atomics (tens of ns each on one address, one after another across
 //     the chip) would set the pace in smaller shares;
-//   * down to kMinGrain otherwise, so that a short queue is spread over all
+//   * down to kMinGrain, one full wave, otherwise, so that a short queue is spread over all
 //     the waves the GPU holds: a wave's items run one sub-batch after another,
 //     each a chain of dependent loads, and with shares of kMaxGrain a
 //     65536-path launch would occupy 256 of 1024 SIMDs for four such chains.
+//     Shares of less than a wave (16 or 32 rays to each traversal wave, on
+//     more waves) are slower: the SIMDs then issue more instructions for the
+//     same rays (Cornell 256x256 at 1 spp 2.9 and 2.4 ms against 2.1).
 // The first share of each home wave is dealt by its index, so a queue that
 // one round of shares covers takes no atomics at all; waves without a share
-// leave at once.  Measured against shares of kMaxGrain from one counter:
-// Cornell 256x256 at 1 spp 6.9 -> 3.1 ms, its 512x512 smoke at 16 spp (23
+// leave at once.  Measured against shares of kMaxGrain from one counter (with
+// 16-ray shares in the traversal kernels): Cornell 256x256 at 1 spp 6.9 -> 3.1 ms, its 512x512 smoke at 16 spp (23
 // passes, the last of them short) 49 -> 40 ms, the interior at 1080p and 1 spp
 // 27.7 -> 24.1 ms, at 64 spp 958 -> 950 ms.
 template <uint32_t kMinGrain, uint32_t kMaxGrain, typename Count, typename Work, typename Body>
@@ -343,6 +346,7 @@ __device__ __forceinline__ void for_slots(const FrameSlot *__restrict__ fs, uint
     {
         uint32_t total = 0;
         for (uint32_t s = 0; s < nfs; ++s) total += count(fs[s]);
+        total = uniform(total);
         if (total == 0) return;
         const uint32_t per = total / gridDim.x;
         const uint32_t grain = per >= kMaxGrain ? kMaxGrain : per <= kMinGrain ? kMinGrain : per / kMinGrain * kMinGrain;
@@ -362,7 +366,7 @@ __device__ __forceinline__ void for_slots(const FrameSlot *__restrict__ fs, uint
     for (uint32_t j = 0; j < nfs; ++j) {
         const uint32_t s = __builtin_amdgcn_readfirstlane(home + j >= nfs ? home + j - nfs : home + j);
         const FrameSlot &f = fs[s];
-        const uint32_t n = count(f);
+        const uint32_t n = uniform(count(f));
         const uint32_t before = s == 0 ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane(w[4]);
         w[4] = before + n;
         if (n == 0) continue;
@@ -592,6 +596,7 @@ __device__ __forceinline__ void extend_body(const DevScene &sc, const PtParams &
     TraceCounters tc{0, 0};
     RefillRange<32> rr(share, cnt + kCtrWorkExtend, cnt[kCtrActive]);
 
+    const TravScene ts(sc);
     Traversal<kModeAll, false, kNearby, true, kSphere, kStack> tv;
     uint32_t p = 0;
     int r = kLaneIdle;
@@ -616,7 +621,7 @@ __device__ __forceinline__ void extend_body(const DevScene &sc, const PtParams &
         for (;;) {
             const uint64_t busy = __ballot(r == kTravContinue);
             if (busy == 0 || (uint32_t)(kBlock - __popcll(busy)) >= want) break;
-            wave_step<16, true>(tv, r, sc, ls, tc);
+            wave_step<16, true>(tv, r, ts, ls, tc);
         }
         if (r != kTravContinue && r != kLaneIdle) {
             if (r == kTravOverflow) atomicOr(prm.error, 1u);
@@ -679,7 +684,7 @@ __device__ __forceinline__ void extend_body(const DevScene &sc, const PtParams &
 template <bool kNearby, bool kMedia, bool kSphere, int kStack>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kSphere ? 1 : 4))) void k_extend_m(const FrameSlot *__restrict__ fs, uint32_t nfs, uint32_t pass)
 {
-    for_slots<kTravGrain, kBlock * kSub>(
+    for_slots<kBlock, kBlock * kSub>(
         fs, nfs, [&](const FrameSlot &f) { return pass_counter(f, pass, kCtrActive); },
         [&](const FrameSlot &f) { return pass_work(f, pass, kCtrWorkExtend); },
         [&](const FrameSlot &f, const Share &share) {
@@ -1581,6 +1586,7 @@ __device__ __forceinline__ void shadow_body(const DevScene &sc, const PtParams &
     RefillRange<16> rr(share, cnt + kCtrWorkShadow, cnt[kCtrShadow]);
 
     // one lane walks its path's recorded rays (slots k) in order
+    const TravScene ts(sc);
     Traversal<kModeSkipBoundary, true, false, true, kSphere, kStack> tv;
     uint32_t p = 0, fl = 0;
     int k = 0;
@@ -1609,7 +1615,7 @@ __device__ __forceinline__ void shadow_body(const DevScene &sc, const PtParams &
         for (;;) {
             const uint64_t busy = __ballot(r == kTravContinue);
             if (busy == 0 || (uint32_t)(kBlock - __popcll(busy)) >= want) break;
-            wave_step<24, false>(tv, r, sc, ls, tc);
+            wave_step<24, false>(tv, r, ts, ls, tc);
         }
         // finished rays: note the result, start the path's next ray or
         // finish the path (a ray can end in init, hence the loop)
@@ -1644,7 +1650,7 @@ __device__ __forceinline__ void shadow_body(const DevScene &sc, const PtParams &
 template <bool kMedia, bool kSphere, int kStack, bool kAdj = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kAdj ? 4 : 5))) void k_shadow_m(const FrameSlot *__restrict__ fs, uint32_t nfs, uint32_t pass)
 {
-    for_slots<kTravGrain, kBlock * kSub>(
+    for_slots<kBlock, kBlock * kSub>(
         fs, nfs, [&](const FrameSlot &f) { return pass_counter(f, pass, kCtrShadow); },
         [&](const FrameSlot &f) { return pass_work(f, pass, kCtrWorkShadow); },
         [&](const FrameSlot &f, const Share &share) {
@@ -1906,7 +1912,7 @@ __global__ void k_tonemap(float4 *img, uint32_t n, float gamma, float exposure)
 
 // ------------------------------------------------------------ launchers
 // Persistent pass kernels: the caller's persistent_waves, or by default one
-// wave per kTravGrain paths of the launch (all slots), at most
+// wave per 64 paths of the launch (all slots), at most
 // kMaxPersistentWaves (the traversal spill area holds kSpillThreads threads);
 // launch_persistent then holds each kernel to the waves the GPU has room for.
 // Waves a queue has no share for leave at once (for_slots).  Every pass kernel
@@ -1915,7 +1921,7 @@ uint32_t persistent_waves(uint64_t paths, uint32_t requested, uint32_t spill_thr
 {
     static_assert(kMaxPersistentWaves * kBlock == kSpillThreads, "one spill row per lane");
     const uint32_t most = spill_threads / kBlock;  // one spill row per lane
-    const uint64_t waves = (paths + kTravGrain - 1) / kTravGrain;
+    const uint64_t waves = (paths + kBlock - 1) / kBlock;
     const uint64_t cap = std::min<uint64_t>(requested ? requested : most, most);
     return (uint32_t)std::max<uint64_t>(std::min(waves, cap), 1);
 }
