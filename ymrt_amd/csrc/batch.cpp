@@ -239,8 +239,8 @@ int render_batch(ymrt_context *ctx, const ymrt_batch_item *items, uint32_t n, ui
             // the round's capacity as their stride)
             PathState ps = rb.ps;
             auto sh = [&](auto *&p, size_t per_path = 1) { p += off * per_path; };
-            sh(ps.ray, 2), sh(ps.bs, 2), sh(ps.L), sh(ps.xhdr), sh(ps.xrec), sh(ps.hit, 2), sh(ps.nb);
-            sh(ps.sh, kShadowSlots * 4), sh(ps.sh_tr), sh(ps.sh_c), sh(ps.sh_flags), sh(ps.out), sh(ps.queue[0]);
+            sh(ps.ray, 2), sh(ps.bs, 2), sh(ps.acc, 2), sh(ps.xhdr), sh(ps.xrec), sh(ps.hit, 2), sh(ps.nb);
+            sh(ps.sh, kShadowSlots * 4), sh(ps.sh_flags), sh(ps.out), sh(ps.queue[0]);
             sh(ps.queue[1]), sh(ps.q_hit), sh(ps.q_hit_vol), sh(ps.q_hit_diffuse), sh(ps.q_hit_metal);
             sh(ps.q_medium), sh(ps.q_shadow), sh(ps.q_transmit), sh(ps.flag), sh(ps.first_hit);
             ps.ccount = rb.ps.ccount + (size_t)s * 4 * ccount_stride;

@@ -55,14 +55,12 @@ inline int layout_buffers(RenderBuffers &rb, size_t n, uint32_t spill_threads, G
     int rc = 0;
     rc |= get(ps.ray, n * 2);
     rc |= get(ps.bs, n * 2);
-    rc |= get(ps.L, n);
+    rc |= get(ps.acc, n * 2);
     rc |= get(ps.xhdr, n);
     rc |= get(ps.xrec, n * kMaxBoundaryRecord);
     rc |= get(ps.hit, n * 2);
     rc |= get(ps.nb, n * 4);
     rc |= get(ps.sh, n * kShadowSlots * 4);
-    rc |= get(ps.sh_tr, n * kShadowSlots);
-    rc |= get(ps.sh_c, n);
     rc |= get(ps.sh_flags, n);
     rc |= get(ps.out, n);
     rc |= get(ps.queue[0], n);

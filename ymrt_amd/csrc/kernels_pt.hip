@@ -471,7 +471,9 @@ __device__ __forceinline__ uint32_t shade_flag(uint32_t cls)
 // shadow flags: bits 0-3 shadow ray k recorded (slots 0-1 shape light,
 // 2-3 distant light), 4-7 ray k crosses the surface, 8-11 ray k reached the
 // light past solid geometry, 12 volume vertex, 13 path ends after this
-// shadow stage, 16-23 vertex depth
+// shadow stage, 16-23 vertex depth, 24-31 and 14-15 the low and high bits of the
+// vertex number (at most kMaxPasses), which keys the random numbers of the
+// transmittance stage
 constexpr uint32_t kShActiveMask = 0xFu;
 constexpr uint32_t kShTransmit0 = 1u << 4;
 constexpr uint32_t kShClear0 = 1u << 8;
@@ -479,6 +481,9 @@ constexpr uint32_t kShClearMask = 0xFu << 8;
 constexpr uint32_t kShVolume = 1u << 12;
 constexpr uint32_t kShTerminate = 1u << 13;
 constexpr uint32_t kShDepthShift = 16;
+static_assert(kMaxPasses < 1024, "a vertex number has ten bits");
+__device__ __forceinline__ uint32_t sh_vertex_bits(uint32_t v) { return (v & 0xFFu) << 24 | ((v >> 8) & 3u) << 14; }
+__device__ __forceinline__ uint32_t sh_vertex(uint32_t fl) { return fl >> 24 | ((fl >> 14) & 3u) << 8; }
 
 // indirect_light_clamp (src/Shading.cu:61-81).  Its powers use the GPU's
 // float powf: the double-precision form (ym_powf) would raise the registers
@@ -546,7 +551,7 @@ __device__ __forceinline__ void raygen_body(const DevScene &sc, const PtParams &
                 *ps.ray_o(p) = f4(cam.position, __uint_as_float(kEmpty));
                 *ps.ray_d(p) = f4(dir, __uint_as_float(kEmpty));
                 *ps.beta(p) = make_float4(1.0f, 1.0f, 1.0f, __uint_as_float(1u | kInfoNeverScatter));
-                ps.L[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                *ps.L(p) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                 store_sampler(ps, p, smp);
                 Transfer t;
                 t.count = cam.record_count;
@@ -645,7 +650,7 @@ __device__ __forceinline__ void extend_body(const DevScene &sc, const PtParams &
             if (pass == 0 && prm.aov) ps.first_hit[p] = hit ? h.inst : kEmpty;
             const bool in_medium = kMedia && prm.media && (gload(ps.xhdr + p) & 0xFFu) != 0;
             if (!hit && !in_medium) {
-                f3 Lv = xyz(gload(ps.L + p));
+                f3 Lv = xyz(gload(ps.L(p)));
                 if (rs.enable_env_light)
                     Lv = Lv + light_clamp(rs, xyz(gload(ps.beta(p))) * background(tv.q.d), info_depth(info));
                 gstore(ps.out + p, f4(Lv, 0.0f));
@@ -917,7 +922,7 @@ __device__ __forceinline__ void medium_body(const DevScene &sc, const PtParams &
                     // every later deposit of the path depends on this flight
                     float scale = 0.0f;
                     if (het && prm.adj.vol != kEmpty) {
-                        const f3 dl = adj_pixel(prm, p) * (xyz(ps.out[p]) - xyz(ps.L[p]));
+                        const f3 dl = adj_pixel(prm, p) * (xyz(ps.out[p]) - xyz(*ps.L(p)));
                         scale = dl.x + dl.y + dl.z;
                     }
                     if (scale != 0.0f) {
@@ -945,7 +950,7 @@ __device__ __forceinline__ void medium_body(const DevScene &sc, const PtParams &
             } else if (hit) {
                 ps.flag[p] = (pass << kFlagBits) | shade_flag(sc.mat_class[sc.instances[ha.y].material]);
             } else {
-                f3 Lv = xyz(ps.L[p]);
+                f3 Lv = xyz(*ps.L(p));
                 if (rs.enable_env_light) Lv = Lv + light_clamp(rs, beta * background(d), info_depth(__float_as_uint(bi.w)));
                 ps.out[p] = f4(Lv, 0.0f);
             }
@@ -1079,7 +1084,7 @@ __device__ __forceinline__ void shade_body(const DevScene &sc, const PtParams &p
             const f3 ray_d = xyz(*ps.ray_d(p));
             f3 beta = xyz(bi);
             Sampler smp = load_sampler(ps, p);
-            ShadowEmit so{ps, p, (uint32_t)depth << kShDepthShift};
+            ShadowEmit so{ps, p, (uint32_t)depth << kShDepthShift | sh_vertex_bits(vertex)};
             bool alive = false;       // a next extension ray
             f3 emitted = s3(0.0f);    // radiance of a light the path ends on
             const f3 sh_beta = beta;
@@ -1308,7 +1313,7 @@ __device__ __forceinline__ void shade_body(const DevScene &sc, const PtParams &p
                         const bool tex_on = A.tex != kEmpty && m.diffuse_albedo_tex == A.tex;
                         rough_entry = A.rough_slot[in.material];
                         if (as >= 0 || tex_on || rough_entry >= 0)
-                            adj_dl = adj_pixel(prm, p) * (xyz(ps.out[p]) - xyz(ps.L[p]));
+                            adj_dl = adj_pixel(prm, p) * (xyz(ps.out[p]) - xyz(*ps.L(p)));
                         if (as >= 0) {
 #pragma unroll
                             for (int c = 0; c < 3; ++c) {
@@ -1461,13 +1466,13 @@ __device__ __forceinline__ void shade_body(const DevScene &sc, const PtParams &p
                 out[0] = true;
                 if (!alive) so.flags |= kShTerminate;
                 ps.sh_flags[p] = so.flags;
-                ps.sh_c[p] = f4(sh_beta, sel_pdf);
+                *ps.sh_c(p) = f4(sh_beta, sel_pdf);
             } else if (!alive) {
                 // the path's radiance changes here only where it ends on a
                 // light; elsewhere it stays in HBM (adding 0 to -0 gives the
                 // same output as the reference's sum: a path's radiance
                 // starts at +0)
-                ps.out[p] = f4(xyz(ps.L[p]) + emitted, 0.0f);
+                ps.out[p] = f4(xyz(*ps.L(p)) + emitted, 0.0f);
             }
             info = (uint32_t)depth | (never_scatter ? kInfoNeverScatter : 0u) | (pending ? kInfoPendingBunch : 0u) |
                    (vertex << 16);
@@ -1476,8 +1481,6 @@ __device__ __forceinline__ void shade_body(const DevScene &sc, const PtParams &p
                 *ps.ray_o(p) = f4(next_o, __uint_as_float(next_li));
                 *ps.ray_d(p) = f4(next_d, __uint_as_float(next_lt));
                 *ps.beta(p) = f4(beta, __uint_as_float(info));
-            } else if (nee) {
-                *ps.info(p) = info;  // the transmittance stage's random numbers are keyed by the vertex
             }
         }
     });
@@ -1504,39 +1507,53 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kGraph ?
 
 // ------------------------------------------------------------ shadow
 // NEE contribution of a path's shadow rays: per light kind, the sum of
-// mis * tr * f * Li over the rays that reached the light, divided by the
-// light-selection pdf, clamped and deposited, distant light first
-// (EvalDistantLight, src/Shading.cu:83-198, then EvalShapeLight 294-417, as
-// the shading stage adds them at 2217-2240).  with_tr: the transmittance of
-// each ray is in sh_tr (paths in media), otherwise 1.  kAdj (the adjoint's
-// replay): at a surface vertex with a target roughness, each ray's deposit D
-// adds adj . D * (g_ray - g_continuation) to that roughness's gradient (the
-// continuation's event counted D with the continuation's factor).
-template <bool kAdj = false>
-__device__ __forceinline__ void shadow_finish(const PtParams &prm, const PathState &ps, uint32_t p, uint32_t fl,
-                                              uint32_t distant_count, bool with_tr, AdjSums<kAdj> *sums = nullptr)
-{
-    const uint32_t cap = prm.cap;
+// mis * tr * f * Li over the rays that reached the light (ShadowSum::add, in
+// slot order within a kind), divided by the light-selection pdf, clamped and
+// deposited (shadow_deposit), distant light first (EvalDistantLight,
+// src/Shading.cu:83-198, then EvalShapeLight 294-417, as the shading stage
+// adds them at 2217-2240).  kAdj (the adjoint's replay): at a surface vertex
+// with a target roughness, each ray's deposit D adds adj . D * (g_ray -
+// g_continuation) to that roughness's gradient (the continuation's event
+// counted D with the continuation's factor).
+template <bool kAdj>
+struct ShadowSum {
     f3 shape = s3(0.0f), dist = s3(0.0f);
-    f3 rc[kShadowSlots];
-    float rg[kShadowSlots];
-    static_for<0, kShadowSlots>([&](auto K) {
-        rc[K()] = s3(0.0f);
-        rg[K()] = 0.0f;
-        if ((fl & (1u << K())) && (fl & (kShClear0 << K()))) {
-            const float4 f4v = ps.shadow(K(), p)[2];
-            const float4 li4 = ps.shadow(K(), p)[3];
-            const f3 tr = with_tr ? xyz(ps.sh_tr[(size_t)K() * cap + p]) : s3(1.0f);
-            const f3 c = ((f4v.w * tr) * xyz(f4v)) * xyz(li4);
-            if (K() < 2) shape = shape + c;
-            else dist = dist + c;
-            if constexpr (kAdj) {
-                rc[K()] = c;
-                rg[K()] = li4.w;
-            }
-        }
-    });
-    const float4 c4 = ps.sh_c[p];
+    f3 rc[kAdj ? kShadowSlots : 1];
+    float rg[kAdj ? kShadowSlots : 1];
+    __device__ __forceinline__ ShadowSum()
+    {
+        if constexpr (kAdj)
+            static_for<0, kShadowSlots>([&](auto K) {
+                rc[K()] = s3(0.0f);
+                rg[K()] = 0.0f;
+            });
+    }
+    // shadow ray k of path p reached its light with transmittance tr; returns
+    // its term
+    __device__ __forceinline__ f3 add(const PathState &ps, uint32_t p, int k, f3 tr)
+    {
+        const float4 f4v = ps.shadow(k, p)[2];
+        const float4 li4 = ps.shadow(k, p)[3];
+        const f3 c = ((f4v.w * tr) * xyz(f4v)) * xyz(li4);
+        if (k < 2) shape = shape + c;
+        else dist = dist + c;
+        if constexpr (kAdj)
+            static_for<0, kShadowSlots>([&](auto K) {
+                if (K() == k) {
+                    rc[K()] = c;
+                    rg[K()] = li4.w;
+                }
+            });
+        return c;
+    }
+};
+
+template <bool kAdj>
+__device__ __forceinline__ void shadow_deposit(const PtParams &prm, const PathState &ps, uint32_t p, uint32_t fl,
+                                               uint32_t distant_count, const ShadowSum<kAdj> &sum,
+                                               AdjSums<kAdj> *sums)
+{
+    const float4 c4 = *ps.sh_c(p);
     const f3 beta = xyz(c4);
     if constexpr (kAdj) {
         if (!(fl & kShVolume)) {
@@ -1547,22 +1564,22 @@ __device__ __forceinline__ void shadow_finish(const PtParams &prm, const PathSta
                 float acc = 0.0f;
                 static_for<0, kShadowSlots>([&](auto K) {
                     const float scale = K() < 2 ? safe_rcp(c4.w) : (float)distant_count;
-                    const f3 d = beta * (rc[K()] * scale);
-                    acc += dot(a, d) * (rg[K()] - gc);
+                    const f3 d = beta * (sum.rc[K()] * scale);
+                    acc += dot(a, d) * (sum.rg[K()] - gc);
                 });
                 sums->roughness(ag.x, acc);
             }
         }
     }
     const int depth = (int)((fl >> kShDepthShift) & 0xFFu);
-    f3 L = xyz(ps.L[p]);
-    if (distant_count > 0) L = L + light_clamp(prm.rs, beta * (dist / (1.0f / (float)distant_count)), depth);
+    f3 L = xyz(*ps.L(p));
+    if (distant_count > 0) L = L + light_clamp(prm.rs, beta * (sum.dist / (1.0f / (float)distant_count)), depth);
     // EvalShapeLight returns direct * SafeRcp(select pdf); the volume variant
     // divides when the pdf is positive.
-    const f3 sel = (fl & kShVolume) ? (c4.w > 0.0f ? shape / c4.w : s3(0.0f)) : shape * safe_rcp(c4.w);
+    const f3 sel = (fl & kShVolume) ? (c4.w > 0.0f ? sum.shape / c4.w : s3(0.0f)) : sum.shape * safe_rcp(c4.w);
     L = L + light_clamp(prm.rs, beta * sel, depth);
-    ps.L[p] = f4(L, 0.0f);
     if (fl & kShTerminate) ps.out[p] = f4(L, 0.0f);
+    else *ps.L(p) = f4(L, 0.0f);
 }
 
 // Any-hit for each shadow ray against non-boundary instances
@@ -1634,7 +1651,11 @@ __device__ __forceinline__ void shadow_body(const DevScene &sc, const PtParams &
                     ps.sh_flags[p] = fl;
                     ps.flag[p] = (pass << kFlagBits) | kFlagTransmit;
                 } else {
-                    shadow_finish<kAdj>(prm, ps, p, fl, sc.distant_count, false, &sums);
+                    ShadowSum<kAdj> sum;
+                    static_for<0, kShadowSlots>([&](auto K) {
+                        if ((fl & (1u << K())) && (fl & (kShClear0 << K()))) sum.add(ps, p, K(), s3(1.0f));
+                    });
+                    shadow_deposit<kAdj>(prm, ps, p, fl, sc.distant_count, sum, &sums);
                 }
             }
         }
@@ -1692,8 +1713,6 @@ __device__ __forceinline__ void transmit_body(const DevScene &sc, const PtParams
             const uint32_t p = ps.q_transmit[i];
             slot = p;
             const uint32_t fl = ps.sh_flags[p];
-            const uint32_t info = *ps.info(p);
-            const uint4 ha = *ps.hit_a(p);
             HashRng rng;
             {
                 // 64-bit like k_raygen: a frame may hold more than 2^32 path slots
@@ -1705,11 +1724,12 @@ __device__ __forceinline__ void transmit_body(const DevScene &sc, const PtParams
                 const uint32_t ty = tile / prm.tiles_x, tx = tile - ty * prm.tiles_x;
                 const uint32_t px = tx * 16u + (within & 15u), py = ty * 16u + (within >> 4);
                 rng.key[0] = py * prm.rs.width + px;
-                rng.key[1] = info_vertex(info);
+                rng.key[1] = sh_vertex(fl);
                 rng.key[2] = s;
                 rng.key[3] = (uint32_t)prm.frame;
                 rng.ctr = 0;
             }
+            ShadowSum<kAdj> sum;
             // distant-light rays first, as the shading stage evaluates them
 #pragma unroll 1
             for (int j = 0; j < kShadowSlots; ++j) {
@@ -1722,15 +1742,16 @@ __device__ __forceinline__ void transmit_body(const DevScene &sc, const PtParams
                     // the vertex's records and nearby list are reloaded per ray
                     // rather than held across the loop (fewer live registers)
                     Transfer t = load_transfer(ps, p, cap);
-                    if (fl & (kShTransmit0 << k)) boundary_bunch(sc, t, load_nearby(ps, p, cap, ha));
-                    const bool volv = (fl & kShVolume) != 0;
+                    if (fl & (kShTransmit0 << k)) boundary_bunch(sc, t, load_nearby(ps, p, cap, *ps.hit_a(p)));
                     Query tq;
                     tq.o = xyz(o4);
                     tq.d = xyz(d4);
                     tq.tmin = kTMin;
                     tq.tmax = o4.w;
-                    tq.last_inst = volv ? kEmpty : ha.y;
-                    tq.last_tri = volv ? kEmpty : ha.z;
+                    // a vertex with shadow rays lies on no boundary (those
+                    // are passed through), so there is no triangle to skip
+                    tq.last_inst = kEmpty;
+                    tq.last_tri = kEmpty;
                     const float maxd = o4.w;
                     float traced = kTMin;
                     int guard = 0;
@@ -1774,14 +1795,11 @@ __device__ __forceinline__ void transmit_body(const DevScene &sc, const PtParams
                 };
                 const uint32_t ctr0 = rng.ctr;
                 const f3 tr = walk(NoTrackEvents{});
-                ps.sh_tr[(size_t)k * cap + p] = f4(tr, 0.0f);
+                const f3 c = sum.add(ps, p, k, tr);
                 if constexpr (kAdj && kHet > 0) {
                     if (prm.adj.vol != kEmpty) {
-                        // this ray's deposit, as shadow_finish sums it
-                        const float4 f4v = ps.shadow(k, p)[2];
-                        const float4 li4 = ps.shadow(k, p)[3];
-                        const float4 c4 = ps.sh_c[p];
-                        const f3 c = ((f4v.w * tr) * xyz(f4v)) * xyz(li4);
+                        // this ray's deposit, as shadow_deposit sums it
+                        const float4 c4 = *ps.sh_c(p);
                         const float scale = k >= 2 ? (float)sc.distant_count
                                             : (fl & kShVolume) ? (c4.w > 0.0f ? 1.0f / c4.w : 0.0f)
                                                                : safe_rcp(c4.w);
@@ -1796,7 +1814,7 @@ __device__ __forceinline__ void transmit_body(const DevScene &sc, const PtParams
                     }
                 }
             }
-            shadow_finish<kAdj>(prm, ps, p, fl, sc.distant_count, true, &sums);
+            shadow_deposit<kAdj>(prm, ps, p, fl, sc.distant_count, sum, &sums);
         }
     });
     sums.end();
@@ -1807,7 +1825,7 @@ __device__ __forceinline__ void transmit_body(const DevScene &sc, const PtParams
 
 
 template <bool kSphere, int kStack, int kHet, bool kAdj = false>
-__global__ __launch_bounds__(kBlock) void k_transmit_m(const FrameSlot *__restrict__ fs, uint32_t nfs, uint32_t pass)
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kHet == 0 ? 3 : kHet == 1 ? 2 : 1))) void k_transmit_m(const FrameSlot *__restrict__ fs, uint32_t nfs, uint32_t pass)
 {
     for_slots<kBlock, kBlock * kSub>(
         fs, nfs, [&](const FrameSlot &f) { return pass_counter(f, pass, kCtrTransmit); },
@@ -1828,7 +1846,7 @@ __device__ __forceinline__ void flush_body(const PtParams &prm, const PathState 
     const uint32_t *q = ps.queue[pass & 1];
     for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
         const uint32_t p = q[i];
-        ps.out[p] = ps.L[p];
+        ps.out[p] = *ps.L(p);
     }
 }
 

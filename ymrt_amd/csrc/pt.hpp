@@ -85,14 +85,12 @@ constexpr int kShadowSlots = 4;
 struct PathState {
     float4 *ray;        // [cap][2] origin and last instance, direction and last triangle
     float4 *bs;         // [cap][2] throughput and info word, sampler
-    float4 *L;
+    float4 *acc;        // [cap][2] radiance so far; throughput at the vertex and light-select pdf of its shadow rays
     uint32_t *xhdr;
     uint4 *xrec;        // [kMaxBoundaryRecord][cap]
     uint4 *hit;         // [cap][2] (t bits, instance, triangle, flags), barycentrics or volume position
     uint2 *nb;          // [4][cap] nearby (instance | back << 31, t bits), lists of more than the hit itself
     float4 *sh;         // [cap][kShadowSlots][4] shadow rays: origin and tmax, direction, f and MIS weight, Li
-    float4 *sh_tr;      // [kShadowSlots][cap] transmittance of shadow rays in media (adjoint replay)
-    float4 *sh_c;       // throughput at the vertex, light-select pdf
     uint32_t *sh_flags;
     float4 *out;        // final radiance per path
     uint32_t *queue[2];
@@ -110,6 +108,8 @@ struct PathState {
     YM_HD float4 *beta(uint32_t p) const { return bs + 2 * (size_t)p; }
     YM_HD uint32_t *info(uint32_t p) const { return reinterpret_cast<uint32_t *>(bs + 2 * (size_t)p) + 3; }
     YM_HD uint4 *smp(uint32_t p) const { return reinterpret_cast<uint4 *>(bs + 2 * (size_t)p + 1); }
+    YM_HD float4 *L(uint32_t p) const { return acc + 2 * (size_t)p; }
+    YM_HD float4 *sh_c(uint32_t p) const { return acc + 2 * (size_t)p + 1; }
     YM_HD uint4 *hit_a(uint32_t p) const { return hit + 2 * (size_t)p; }
     YM_HD float4 *hit_b(uint32_t p) const { return reinterpret_cast<float4 *>(hit + 2 * (size_t)p + 1); }
     // shadow ray k: o, d, f, li at [0..3]
