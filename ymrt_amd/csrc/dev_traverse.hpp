@@ -224,8 +224,11 @@ YM_HD int tri_hit_back(const DevScene &sc, uint32_t inst, uint32_t tri, f3 d)
 // constants and axis) is parked in LDS [kPreSlots][kBlock] when a traversal
 // enters an instance and read back when it leaves, instead of being
 // recomputed with six divisions.
+//
+// With kDeep > 0 the deeper entries go to a private array of kDeep instead of
+// the spill area (for kernels that own no memory).
 constexpr int kPreSlots = 7;
-template <int kBlock, int kWindow = 0, bool kPreLds = false>
+template <int kBlock, int kWindow = 0, bool kPreLds = false, int kDeep = 0>
 struct LaneScratch {
     static constexpr int kLanes = kBlock;
     static constexpr bool kParkPre = kPreLds;
@@ -237,6 +240,7 @@ struct LaneScratch {
     uint32_t *spill;        // global [kMaxSpill][spill_stride], unused when kWindow == 0
     uint32_t spill_stride, spill_index;
     float *pre_park = nullptr;  // LDS [kPreSlots][kBlock] when kPreLds
+    uint32_t deep[kDeep > 0 ? kDeep : 1];
 
     YM_HD void park_pre(const RayPre &r)
     {
@@ -285,7 +289,10 @@ struct LaneScratch {
         } else {
             static_assert((kWindow & (kWindow - 1)) == 0, "window must be a power of two");
             const int w = (sp & (kWindow - 1)) * kBlock + lane;
-            if (sp >= kWindow) gstore(spill + (size_t)(sp - kWindow) * spill_stride + spill_index, stack[w]);
+            if (sp >= kWindow) {
+                if constexpr (kDeep > 0) deep[sp - kWindow] = stack[w];
+                else gstore(spill + (size_t)(sp - kWindow) * spill_stride + spill_index, stack[w]);
+            }
             stack[w] = v;
         }
     }
@@ -297,7 +304,10 @@ struct LaneScratch {
         } else {
             const int w = (sp & (kWindow - 1)) * kBlock + lane;
             const uint32_t v = stack[w];
-            if (sp >= kWindow) stack[w] = gload(spill + (size_t)(sp - kWindow) * spill_stride + spill_index);
+            if (sp >= kWindow) {
+                if constexpr (kDeep > 0) stack[w] = deep[sp - kWindow];
+                else stack[w] = gload(spill + (size_t)(sp - kWindow) * spill_stride + spill_index);
+            }
             return v;
         }
     }
