@@ -1,5 +1,6 @@
 """Chunks of up to 65536 path slots are compacted by one launch, longer ones by
-three.  path_capacity sets the chunk, so the same frame runs through either;
+three; up to 262144 paths share one shading launch, longer ones get one per
+class.  path_capacity sets the chunk, so the same frame runs through either;
 its image must not change, at chunks around a block's 1024 slots, the bound
 and odd pixel counts."""
 import pytest
@@ -10,7 +11,7 @@ from ymrt_amd import abi, scenes
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("w,h,spp", [(67, 45, 23), (272, 256, 1)])
+@pytest.mark.parametrize("w,h,spp", [(67, 45, 23), (272, 256, 1), (264, 256, 4)])
 def test_chunk_sizes_keep_the_frame(gpu_ctx, w, h, spp):
     import torch
     sc = ymrt_amd.Scene(gpu_ctx, scenes.cornell_media(w, h, grid=False))

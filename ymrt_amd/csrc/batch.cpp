@@ -41,7 +41,7 @@ int launch_multi_medium(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v
                         hipStream_t s);
 // mode: 0 free flight, 1 shading, 2 transmittance
 int launch_multi_compact(const FrameSlot *fs, uint32_t nfs, uint32_t blocks, uint32_t pass, int mode, hipStream_t s);
-int launch_multi_shade(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v, bool volume, uint32_t waves,
+int launch_multi_shade(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v, uint64_t paths, uint32_t waves,
                        uint32_t pass, hipStream_t s);
 int launch_multi_shadow(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v, uint32_t waves, uint32_t pass,
                         hipStream_t s);
@@ -258,7 +258,8 @@ int render_batch(ymrt_context *ctx, const ymrt_batch_item *items, uint32_t n, ui
         }
         YM_HIP(hipMemcpyAsync(rb.slots, mem.h_table, sizeof(FrameSlot) * nfs, hipMemcpyHostToDevice, stream));
         YM_HIP(hipMemsetAsync(rb.counters, 0, sizeof(uint32_t) * kCountersPerSlot * nfs, stream));
-        // one wave per 256 paths of the round, within [1024, the spill area]
+        // one wave per 64 paths of the round, within the spill area
+        uint64_t live = paths;  // no fewer than the paths still on their way
         const uint32_t waves = persistent_waves(paths, 0, rb.ps.spill_threads);
         const FrameSlot *fs = rb.slots;
         int rc;
@@ -271,8 +272,7 @@ int render_batch(ymrt_context *ctx, const ymrt_batch_item *items, uint32_t n, ui
                 if ((rc = launch_multi_medium(fs, nfs, v, waves, pass, stream))) return rc;
             }
             if ((rc = launch_multi_compact(fs, nfs, compact_blocks, pass, 1, stream))) return rc;
-            if ((rc = launch_multi_shade(fs, nfs, v, false, waves, pass, stream))) return rc;
-            if (v.media && (rc = launch_multi_shade(fs, nfs, v, true, waves, pass, stream))) return rc;
+            if ((rc = launch_multi_shade(fs, nfs, v, live, waves, pass, stream))) return rc;
             if ((rc = launch_multi_shadow(fs, nfs, v, waves, pass, stream))) return rc;
             if (v.media) {
                 if ((rc = launch_multi_compact(fs, nfs, compact_blocks, pass, 2, stream))) return rc;
@@ -285,6 +285,7 @@ int render_batch(ymrt_context *ctx, const ymrt_batch_item *items, uint32_t n, ui
                 YM_HIP(hipMemcpyAsync(&active, mem.d_active, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
                 YM_HIP(hipStreamSynchronize(stream));
                 if (active == 0) break;
+                live = active;
                 if (pass >= kMaxPasses) {
                     if ((rc = launch_multi_flush(fs, nfs, pass, stream))) return rc;
                     break;

@@ -77,14 +77,14 @@ struct Share {
 
 // Persistent loop over n items (one wave per block): body(i, p, out) handles
 // item i < n, sets p (the path slot it appends) and out[q] for each output
-// queue q.  Survivors of a fetch's sub-batches (at most kS) are staged in LDS and then published with one atomic per queue and
+// queue q.  stage: LDS of kQueues * kS * 64 words.  Survivors of a fetch's
+// sub-batches (at most kS) are staged in LDS and then published with one atomic per queue and
 // a coalesced copy.
 template <int kQueues, int kS = kSub, typename Body>
-__device__ __forceinline__ void run_items(const Share &share, uint32_t *fetch, uint32_t n, uint32_t *const *counters,
-                                          uint32_t *const *queues, Body &&body)
+__device__ __forceinline__ void run_items(uint32_t *stage, const Share &share, uint32_t *fetch, uint32_t n,
+                                          uint32_t *const *counters, uint32_t *const *queues, Body &&body)
 {
     constexpr int kQ = kQueues > 0 ? kQueues : 1;
-    __shared__ uint32_t stage[kQ * kS * kBlock];
     const uint64_t below = (1ull << lane_id()) - 1ull;
     uint32_t base = share.first, end = share.first_end;
     for (;;) {
@@ -329,29 +329,32 @@ __device__ __forceinline__ uint32_t *pass_work(const FrameSlot &f, uint32_t pass
 //     same rays (Cornell 256x256 at 1 spp 2.9 and 2.4 ms against 2.1).
 // The first share of each home wave is dealt by its index, so a queue that
 // one round of shares covers takes no atomics at all; waves without a share
-// leave at once.  Measured against shares of kMaxGrain from one counter (with
+// leave at once.  rot: the grid index of the first wave that takes a share; the
+// waves used come back, so that a kernel with several queues can deal each to
+// other waves.  Measured against shares of kMaxGrain from one counter (with
 // 16-ray shares in the traversal kernels): Cornell 256x256 at 1 spp 6.9 -> 3.1 ms, its 512x512 smoke at 16 spp (23
 // passes, the last of them short) 49 -> 40 ms, the interior at 1080p and 1 spp
 // 27.7 -> 24.1 ms, at 64 spp 958 -> 950 ms.
 template <uint32_t kMinGrain, uint32_t kMaxGrain, typename Count, typename Work, typename Body>
-__device__ __forceinline__ void for_slots(const FrameSlot *__restrict__ fs, uint32_t nfs, Count count, Work work,
-                                          Body body)
+__device__ __forceinline__ uint32_t for_slots(const FrameSlot *__restrict__ fs, uint32_t nfs, Count count, Work work,
+                                              Body body, uint32_t rot = 0)
 {
     // words of Share, then what the next slot's deal needs: kept out of
     // registers while a body runs
     __shared__ uint32_t words[kShareWords];
     LdsWord *w = (LdsWord *)words;
-    const uint32_t me = blockIdx.x;
-    uint32_t home = 0;
+    const uint32_t me = blockIdx.x >= rot ? blockIdx.x - rot : blockIdx.x + gridDim.x - rot;
+    uint32_t home = 0, waves_used;
     {
         uint32_t total = 0;
         for (uint32_t s = 0; s < nfs; ++s) total += count(fs[s]);
         total = uniform(total);
-        if (total == 0) return;
+        if (total == 0) return 0;
         const uint32_t per = total / gridDim.x;
         const uint32_t grain = per >= kMaxGrain ? kMaxGrain : per <= kMinGrain ? kMinGrain : per / kMinGrain * kMinGrain;
         const uint32_t waves = min((total + grain - 1) / grain, gridDim.x);
-        if (me >= waves) return;
+        if (me >= waves) return waves;
+        waves_used = waves;
         // wave w's home is the slot whose items hold item floor(w * total / waves)
         uint32_t before = 0;
         if (nfs > 1) {
@@ -391,6 +394,7 @@ __device__ __forceinline__ void for_slots(const FrameSlot *__restrict__ fs, uint
         }
         body(f, share);
     }
+    return waves_used;
 }
 
 // ------------------------------------------------------------ state access
@@ -508,7 +512,8 @@ __device__ __forceinline__ void raygen_body(const DevScene &sc, const PtParams &
     uint32_t *cnt = prm.counters;  // pass 0 slots
     uint32_t *const ctrs[1] = {cnt + kCtrActive};
     uint32_t *const qs[1] = {ps.queue[0]};
-    run_items<1, kRaygenSub>(share, cnt + kCtrWorkRaygen, prm.chunk_paths, ctrs, qs,
+    __shared__ uint32_t stage[kRaygenSub * kBlock];
+    run_items<1, kRaygenSub>(stage, share, cnt + kCtrWorkRaygen, prm.chunk_paths, ctrs, qs,
                              [&](uint32_t p, uint32_t &slot, bool(&out)[1]) {
         slot = p;
         ps.flag[p] = 0;
@@ -956,7 +961,7 @@ __device__ __forceinline__ void medium_body(const DevScene &sc, const PtParams &
     uint32_t *cnt = prm.counters + pass * kCtrStride;
     const uint32_t n = cnt[kCtrMedium];
     const ymrt_render_settings &rs = prm.rs;
-    run_items<0, kMediumSub>(share, cnt + kCtrWorkMedium, n, nullptr, nullptr, [&](uint32_t i, uint32_t &p, bool(&)[1]) {
+    run_items<0, kMediumSub>(nullptr, share, cnt + kCtrWorkMedium, n, nullptr, nullptr, [&](uint32_t i, uint32_t &p, bool(&)[1]) {
         {
             p = ps.q_medium[i];
             const uint4 ha = *ps.hit_a(p);
@@ -1107,13 +1112,19 @@ __device__ __forceinline__ float shadow_tmax(f3 pos, f3 ldir, f3 lpos, f3 lerr, 
 // faster on the interior frame; 4 waves spill too much).
 // kAdj: the adjoint's replay pass (surface vertices): albedo, texel and
 // roughness gradient events.
+//
+// LDS of a shading wave: the output queues' stage, the texture graph's value
+// stack and the adjoint's sums.
+struct ShadeLds {
+    uint32_t *stage;
+    float *tex, *adj;
+};
+
 template <bool kVolume, bool kGraph, uint32_t kClass = kMatGeneral, bool kAdj = false>
-__device__ __forceinline__ void shade_body(const DevScene &sc, const PtParams &prm, const PathState &ps, uint32_t pass,
-                                           const Share &share)
+__device__ __forceinline__ void shade_body(const ShadeLds &lds, const DevScene &sc, const PtParams &prm,
+                                           const PathState &ps, uint32_t pass, const Share &share)
 {
-    __shared__ float tex_stk[(kVolume || !kGraph) ? 1 : kTexStack * 3 * kBlock];
-    __shared__ float adj_lds[kAdj ? kAdjLds : 1];
-    AdjSums<kAdj> sums{adj_lds, &prm.adj};
+    AdjSums<kAdj> sums{lds.adj, &prm.adj};
     sums.begin();
     uint32_t *cnt = prm.counters + pass * kCtrStride;
     uint32_t *cnt_next = prm.counters + (pass + 1) * kCtrStride;
@@ -1127,7 +1138,7 @@ __device__ __forceinline__ void shade_body(const DevScene &sc, const PtParams &p
     constexpr uint32_t kLobes = kDiffuse ? 1u << kSlotDiffuse
                                 : kMetal ? (1u << kSlotMetal) | (1u << kSlotDiffuse)
                                          : 0u;
-    run_items<2>(share, cnt + (kVolume     ? kCtrWorkShadeVol
+    run_items<2>(lds.stage, share, cnt + (kVolume     ? kCtrWorkShadeVol
                         : kDiffuse ? kCtrWorkShadeDiffuse
                         : kMetal   ? kCtrWorkShadeMetal
                                    : kCtrWorkShade),
@@ -1352,7 +1363,7 @@ __device__ __forceinline__ void shade_body(const DevScene &sc, const PtParams &p
                     const bool is_default = mtype == YMRT_MATERIAL_DEFAULT;
                     const uint32_t normal_tex = kGraph && is_default ? m.normal_mapping_tex : kEmpty;
                     const uint32_t bump_tex = kGraph && is_default && normal_tex == kEmpty ? m.bump_mapping_tex : kEmpty;
-                    TexEval<kGraph> tx{sc, TexCoord{uv, pos, pos_obj}, tex_stk, (int)lane_id()};
+                    TexEval<kGraph> tx{sc, TexCoord{uv, pos, pos_obj}, lds.tex, (int)lane_id()};
                     float4 duv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                     if (bump_tex != kEmpty)
                         duv = camera_uv_differentials(sc.camera, pos, sn, ng, dpdu, dpdv, rs.width, rs.height, 0.25f,
@@ -1549,19 +1560,47 @@ __device__ __forceinline__ void shade_body(const DevScene &sc, const PtParams &p
 }
 
 
-template <bool kVolume, bool kGraph, uint32_t kClass = kMatGeneral, bool kAdj = false>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kGraph ? 2 : 3))) void k_shade_m(const FrameSlot *__restrict__ fs, uint32_t nfs, uint32_t pass)
+template <bool kVolume, bool kGraph, uint32_t kClass, bool kAdj>
+__device__ __forceinline__ uint32_t shade_class(const ShadeLds &lds, const FrameSlot *__restrict__ fs, uint32_t nfs,
+                                                uint32_t pass, uint32_t rot)
 {
     constexpr uint32_t kQueue = kVolume ? kCtrHitVol : kClass == kMatDiffuse ? kCtrHitDiffuse
                                 : kClass == kMatMetal ? kCtrHitMetal : kCtrHit;
     constexpr uint32_t kWork = kVolume ? kCtrWorkShadeVol : kClass == kMatDiffuse ? kCtrWorkShadeDiffuse
                                : kClass == kMatMetal ? kCtrWorkShadeMetal : kCtrWorkShade;
-    for_slots<kBlock, kBlock * kSub>(
+    const uint32_t used = for_slots<kBlock, kBlock * kSub>(
         fs, nfs, [&](const FrameSlot &f) { return pass_counter(f, pass, kQueue); },
         [&](const FrameSlot &f) { return pass_work(f, pass, kWork); },
         [&](const FrameSlot &f, const Share &share) {
-            shade_body<kVolume, kGraph, kClass, kAdj>(f.sc, f.prm, f.ps, pass, share);
-        });
+            shade_body<kVolume, kGraph, kClass, kAdj>(lds, f.sc, f.prm, f.ps, pass, share);
+        },
+        rot);
+    return (rot + used) % gridDim.x;
+}
+
+// One shading class per launch.
+template <bool kVolume, bool kGraph, uint32_t kClass = kMatGeneral, bool kAdj = false>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kGraph ? 2 : 3))) void k_shade_m(const FrameSlot *__restrict__ fs, uint32_t nfs, uint32_t pass)
+{
+    __shared__ uint32_t stage[2 * kSub * kBlock];
+    __shared__ float tex_stk[kGraph && !kVolume ? kTexStack * 3 * kBlock : 1];
+    __shared__ float adj_lds[kAdj ? kAdjLds : 1];
+    shade_class<kVolume, kGraph, kClass, kAdj>(ShadeLds{stage, tex_stk, adj_lds}, fs, nfs, pass, 0);
+}
+
+// All shading classes of a pass of short queues in one launch, and with kMedia
+// the volume vertices.  Launched one after another, each class is a chain of
+// dependent loads of 25-35 us on a queue that leaves most of the GPU idle;
+// here a class' waves are others than those the classes before it took.
+template <bool kMedia>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_shade_all_m(const FrameSlot *__restrict__ fs, uint32_t nfs, uint32_t pass)
+{
+    __shared__ uint32_t stage[2 * kSub * kBlock];
+    const ShadeLds lds{stage, nullptr, nullptr};
+    uint32_t rot = shade_class<false, false, kMatGeneral, false>(lds, fs, nfs, pass, 0);
+    rot = shade_class<false, false, kMatMetal, false>(lds, fs, nfs, pass, rot);
+    rot = shade_class<false, false, kMatDiffuse, false>(lds, fs, nfs, pass, rot);
+    if constexpr (kMedia) shade_class<true, false, kMatGeneral, false>(lds, fs, nfs, pass, rot);
 }
 
 
@@ -1769,7 +1808,7 @@ __device__ __forceinline__ void transmit_body(const DevScene &sc, const PtParams
     __shared__ float adj_lds[kAdj ? kAdjLds : 1];
     AdjSums<kAdj> sums{adj_lds, &prm.adj};
     sums.begin();
-    run_items<0>(share, cnt + kCtrWorkTransmit, n, nullptr, nullptr, [&](uint32_t i, uint32_t &slot, bool(&)[1]) {
+    run_items<0>(nullptr, share, cnt + kCtrWorkTransmit, n, nullptr, nullptr, [&](uint32_t i, uint32_t &slot, bool(&)[1]) {
         {
             const uint32_t p = ps.q_transmit[i];
             slot = p;
@@ -2134,13 +2173,30 @@ static void shade_m(const FrameSlot *fs, uint32_t nfs, uint32_t waves, uint32_t 
     launch_persistent((k_shade_m<false, kGraph, kMatMetal, kAdj>), waves, s, fs, nfs, pass);
 }
 
-int launch_multi_shade(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v, bool volume, uint32_t waves,
+// With up to this many paths the shading classes share one launch (frames
+// without texture graphs; not the adjoint's replay).  One launch against one
+// per class, ms per frame at 2^16, 2^18, 2^19 and 2^21 paths: Cornell 1.64 and
+// 2.01, 2.94 and 3.34, 4.56 and 4.89, 8.92 and 8.97; outdoor with fog 3.13 and
+// 4.21, 4.97 and 5.98, 6.59 and 7.39, 12.9 and 12.8; smoke 5.48 and 6.67, 8.21
+// and 9.26, 11.4 and 11.9, 28.9 and 27.4; interior 3.89 and 4.22, 6.24 and
+// 6.47, 10.6 and 10.0, 21.1 and 20.6.  Long queues lose: their waves run
+// different classes at once, which share an instruction cache.
+constexpr uint64_t kShadeAllPaths = 1u << 18;
+
+// paths: no fewer than the launch's queues hold together.
+int launch_multi_shade(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v, uint64_t paths, uint32_t waves,
                        uint32_t pass, hipStream_t s)
 {
-    // volume vertices carry no adjoint events of their own
-    if (volume) launch_persistent((k_shade_m<true, false>), waves, s, fs, nfs, pass);
-    else if (v.graph) v.adj ? shade_m<true, true>(fs, nfs, waves, pass, s) : shade_m<true, false>(fs, nfs, waves, pass, s);
+    if (paths <= kShadeAllPaths && !v.graph && !v.adj) {
+        if (v.media) launch_persistent(k_shade_all_m<true>, waves, s, fs, nfs, pass);
+        else launch_persistent(k_shade_all_m<false>, waves, s, fs, nfs, pass);
+        YM_HIP(hipGetLastError());
+        return YMRT_OK;
+    }
+    if (v.graph) v.adj ? shade_m<true, true>(fs, nfs, waves, pass, s) : shade_m<true, false>(fs, nfs, waves, pass, s);
     else v.adj ? shade_m<false, true>(fs, nfs, waves, pass, s) : shade_m<false, false>(fs, nfs, waves, pass, s);
+    // volume vertices carry no adjoint events of their own
+    if (v.media) launch_persistent((k_shade_m<true, false>), waves, s, fs, nfs, pass);
     YM_HIP(hipGetLastError());
     return YMRT_OK;
 }

@@ -28,7 +28,7 @@ int launch_multi_medium(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v
                         hipStream_t s);
 // mode: 0 free flight, 1 shading, 2 transmittance
 int launch_multi_compact(const FrameSlot *fs, uint32_t nfs, uint32_t blocks, uint32_t pass, int mode, hipStream_t s);
-int launch_multi_shade(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v, bool volume, uint32_t waves,
+int launch_multi_shade(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v, uint64_t paths, uint32_t waves,
                        uint32_t pass, hipStream_t s);
 int launch_multi_shadow(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v, uint32_t waves, uint32_t pass,
                         hipStream_t s);
@@ -288,6 +288,7 @@ static int run_frame(ymrt_scene *sc, RenderBuffers *rb, uint32_t chunk_paths_max
         if ((r = timed(st(0), [&] { return launch_multi_raygen(f, 1, waves, stream); }))) return r;
         uint32_t pass = 0;
         uint32_t next_check = (uint32_t)rs->ray_depth + 1;
+        uint64_t live = prm.chunk_paths;  // no fewer than the paths still on their way
         for (;;) {
             if ((r = timed(st(1), [&] { return launch_multi_extend(f, 1, vv, waves, pass, stream); }))) return r;
             if (media && (r = timed(st(5), [&] {
@@ -296,8 +297,7 @@ static int run_frame(ymrt_scene *sc, RenderBuffers *rb, uint32_t chunk_paths_max
                           })))
                 return r;
             if ((r = timed(st(2), [&] { return launch_multi_compact(f, 1, blocks, pass, 1, stream); }))) return r;
-            if ((r = timed(st(2), [&] { return launch_multi_shade(f, 1, vv, false, waves, pass, stream); }))) return r;
-            if (media && (r = timed(st(2), [&] { return launch_multi_shade(f, 1, vv, true, waves, pass, stream); })))
+            if ((r = timed(st(2), [&] { return launch_multi_shade(f, 1, vv, live, waves, pass, stream); })))
                 return r;
             if ((r = timed(st(3), [&] { return launch_multi_shadow(f, 1, vv, waves, pass, stream); }))) return r;
             if (media && (r = timed(st(6), [&] {
@@ -312,6 +312,7 @@ static int run_frame(ymrt_scene *sc, RenderBuffers *rb, uint32_t chunk_paths_max
                                       hipMemcpyDeviceToHost, stream));
                 YM_HIP(hipStreamSynchronize(stream));
                 if (active == 0) break;
+                live = active;
                 if (pass >= kMaxPasses) {
                     if ((r = launch_multi_flush(f, 1, pass, stream))) return r;
                     break;
