@@ -253,11 +253,11 @@ typedef struct ymrt_render_settings {
     float exposure;
     uint32_t path_capacity;          /* paths in flight per chunk; 0: up to 64 M,
                                         within a quarter of free device memory
-                                        (about 720 B per path)                */
+                                        (at most 720 B per path)              */
     uint32_t persistent_waves;       /* waves of each persistent pass kernel,
                                         at most 5120 (the traversal spill
-                                        area); 0: one per 256 paths of the
-                                        chunk, within [1024, 5120].  Each
+                                        area); 0: one per 64 paths of the
+                                        chunk, at most 5120.  Each
                                         kernel launches at most the waves the
                                         GPU holds of it at once.  Like
                                         path_capacity it changes no pixel.    */

@@ -17,7 +17,7 @@
 
 namespace ym {
 
-// 64 MiB: 65536 paths of path state (about 656 B each) and the traversal
+// 64 MiB: 65536 paths of path state (about 580 B each) and the traversal
 // spill rows of 1024 waves (48 entries x 4 B per lane).
 constexpr size_t kNoAllocScratchBytes = size_t(64) << 20;
 constexpr uint32_t kNoAllocPaths = 1u << 16;

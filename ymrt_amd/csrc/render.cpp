@@ -3,8 +3,8 @@
 // Replaces RenderModule::PathTracingExecuteTask (src/core/RenderModule.cpp:494-653).
 // The reference regenerates paths into a 1M-ray queue and round-trips three
 // counters through the host after every stage (8 synchronisations per batch).
-// Here the frame is cut into chunks of whole pixels (capacity paths each, 4M
-// by default: ~1.2 GB of state, a sliver of the 288 GB HBM); each chunk runs
+// Here the frame is cut into chunks of whole pixels (capacity paths each, up
+// to 64 M by default, within a quarter of the free memory); each chunk runs
 // raygen, then extend/shade/shadow passes whose queue lengths live in device
 // counters, then a resolve into the noise image.  The host reads one counter
 // per chunk, after ray_depth + 1 passes, to decide whether boundary
@@ -394,7 +394,9 @@ static int run_frame(ymrt_scene *sc, RenderBuffers *rb, uint32_t chunk_paths_max
             stats->launches_transmit = launches[6];
             stats->ms_adjoint = ms[7];
             stats->launches_extend = launches[1];
-            stats->launches_shade = launches[2];
+            // a pass of a scene with media counts its volume vertices as a
+            // launch of their own, also where they share one with the surfaces
+            stats->launches_shade = launches[2] + (media ? launches[1] : 0u);
             stats->launches_shadow = launches[3];
             float tot = 0.0f;
             YM_HIP(hipEventElapsedTime(&tot, frame_a, frame_b));
