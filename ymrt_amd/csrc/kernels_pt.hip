@@ -1592,14 +1592,15 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kGraph ?
 // the volume vertices.  Launched one after another, each class is a chain of
 // dependent loads of 25-35 us on a queue that leaves most of the GPU idle;
 // here a class' waves are others than those the classes before it took.
-template <bool kMedia>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_shade_all_m(const FrameSlot *__restrict__ fs, uint32_t nfs, uint32_t pass)
+template <bool kMedia, bool kGraph = false>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kGraph ? 2 : 3))) void k_shade_all_m(const FrameSlot *__restrict__ fs, uint32_t nfs, uint32_t pass)
 {
     __shared__ uint32_t stage[2 * kSub * kBlock];
-    const ShadeLds lds{stage, nullptr, nullptr};
-    uint32_t rot = shade_class<false, false, kMatGeneral, false>(lds, fs, nfs, pass, 0);
-    rot = shade_class<false, false, kMatMetal, false>(lds, fs, nfs, pass, rot);
-    rot = shade_class<false, false, kMatDiffuse, false>(lds, fs, nfs, pass, rot);
+    __shared__ float tex_stk[kGraph ? kTexStack * 3 * kBlock : 1];
+    const ShadeLds lds{stage, tex_stk, nullptr};
+    uint32_t rot = shade_class<false, kGraph, kMatGeneral, false>(lds, fs, nfs, pass, 0);
+    rot = shade_class<false, kGraph, kMatMetal, false>(lds, fs, nfs, pass, rot);
+    rot = shade_class<false, kGraph, kMatDiffuse, false>(lds, fs, nfs, pass, rot);
     if constexpr (kMedia) shade_class<true, false, kMatGeneral, false>(lds, fs, nfs, pass, rot);
 }
 
@@ -2173,20 +2174,28 @@ static void shade_m(const FrameSlot *fs, uint32_t nfs, uint32_t waves, uint32_t 
     launch_persistent((k_shade_m<false, kGraph, kMatMetal, kAdj>), waves, s, fs, nfs, pass);
 }
 
-// With up to this many paths the shading classes share one launch (frames
-// without texture graphs; not the adjoint's replay).  One launch against one
+// With up to this many paths the shading classes share one launch (not in the
+// adjoint's replay, nor in frames with texture graphs and media).  One launch against one
 // per class, ms per frame at 2^16, 2^18, 2^19 and 2^21 paths: Cornell 1.64 and
 // 2.01, 2.94 and 3.34, 4.56 and 4.89, 8.92 and 8.97; outdoor with fog 3.13 and
 // 4.21, 4.97 and 5.98, 6.59 and 7.39, 12.9 and 12.8; smoke 5.48 and 6.67, 8.21
 // and 9.26, 11.4 and 11.9, 28.9 and 27.4; interior 3.89 and 4.22, 6.24 and
 // 6.47, 10.6 and 10.0, 21.1 and 20.6.  Long queues lose: their waves run
-// different classes at once, which share an instruction cache.
+// different classes at once, which share an instruction cache.  Frames with
+// texture graphs and no media share one launch at any length: their general
+// class takes most of the time, and the others then fill the lanes and waves
+// it leaves at its end (procedural box, 4.9 M paths: 17.8 -> 17.2 ms).
 constexpr uint64_t kShadeAllPaths = 1u << 18;
 
 // paths: no fewer than the launch's queues hold together.
 int launch_multi_shade(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v, uint64_t paths, uint32_t waves,
                        uint32_t pass, hipStream_t s)
 {
+    if (v.graph && !v.media && !v.adj) {
+        launch_persistent((k_shade_all_m<false, true>), waves, s, fs, nfs, pass);
+        YM_HIP(hipGetLastError());
+        return YMRT_OK;
+    }
     if (paths <= kShadeAllPaths && !v.graph && !v.adj) {
         if (v.media) launch_persistent(k_shade_all_m<true>, waves, s, fs, nfs, pass);
         else launch_persistent(k_shade_all_m<false>, waves, s, fs, nfs, pass);
