@@ -428,7 +428,7 @@ def main():
                                        "FETCH_SIZE + WRITE_SIZE per extension ray (8 spp run of this scene), "
                                        "times this run's extension rays per launch" if traffic else None,
                      "physical_frac": round(physical / HBM_PEAK_GBS, 4) if physical else None,
-                     "limiter": "not HBM: nodes and triangles come from L2/MALL (physical bytes are a sixth of "
+                     "limiter": "not HBM: nodes and triangles come from L2/MALL (physical bytes are a fifth of "
                                 "the algorithmic ones); the kernel is bound by VALU issue under divergence and "
                                 "dependent-load latency (SQ counters in profiles/traversal_shading_sq_counters.md)",
                      "bytes_per_launch": int(dom_bytes / max(dom_launch, 1)),
