@@ -226,7 +226,10 @@ YM_HD int tri_hit_back(const DevScene &sc, uint32_t inst, uint32_t tri, f3 d)
 // recomputed with six divisions.
 //
 // With kDeep > 0 the deeper entries go to a private array of kDeep instead of
-// the spill area (for kernels that own no memory).
+// the spill area (for kernels that own no memory).  The kernel declares the
+// array beside this struct: an array indexed at run time inside it would keep
+// the whole struct in private memory, and every step would load its pointers
+// and the lane from there.
 constexpr int kPreSlots = 7;
 template <int kBlock, int kWindow = 0, bool kPreLds = false, int kDeep = 0>
 struct LaneScratch {
@@ -240,7 +243,7 @@ struct LaneScratch {
     uint32_t *spill;        // global [kMaxSpill][spill_stride], unused when kWindow == 0
     uint32_t spill_stride, spill_index;
     float *pre_park = nullptr;  // LDS [kPreSlots][kBlock] when kPreLds
-    uint32_t deep[kDeep > 0 ? kDeep : 1];
+    uint32_t *deep = nullptr;   // private [kDeep]
 
     YM_HD void park_pre(const RayPre &r)
     {

@@ -2,7 +2,7 @@
 // sampler probes behind ymrt_trace_* / ymrt_halton_* in include/ymrt.h.
 //
 // One traversal per lane, 64-lane workgroups (one wave64 each), the traversal
-// stack in LDS.  A ray is read as two 16-B loads and its hit written as one
+// stack or its top in LDS.  A ray is read as two 16-B loads and its hit written as one
 // 16-B store.
 #include <algorithm>
 
@@ -20,31 +20,55 @@ constexpr int kTraceBlock = 64;
 // node-first rule of the path tracer's traversal kernels.
 constexpr uint32_t kTraceWaves = 4096;
 constexpr int kTraceIdle = 3;
-// With kDeep, kTraceWindow stack entries per lane are in LDS and the deeper
-// ones (rare) in private memory: the whole stack in LDS, 12 to 24 KB per wave,
-// holds a CU to 13 to 6 waves where the registers allow 16 to 20 (4 M
-// closest-hit rays against 2 M triangles 1765 -> 1588 us, 1 M any-hit rays
-// against 500 k 473 -> 425 us).  Calls of up to one wave per SIMD and stacks
-// of 32 entries stay in LDS: LDS is no limit there, and a kernel with private
-// memory starts later (4095 rays 68 us against 72).
-constexpr int kTraceWindow = 16;
-constexpr uint32_t kTraceShallowWaves = 1024;
 
-template <bool kAny, bool kCount, bool kSphere, int kStack, bool kDeep>
+// Where a ray's stack lives.  The whole stack in LDS (kWindow 0) is the form
+// with the fewest instructions per step, but 48 entries take 13.75 KB per wave,
+// which holds a CU to 11 waves (64 entries 9, 96 entries 6) where the registers
+// allow 16 to 20.  Calls whose waves are all resident that way use it, and so
+// do all calls on stacks of 32 entries, of which a CU holds 16 waves.  Other
+// calls keep kWindow entries per lane in LDS and the deeper ones, which few
+// rays reach, in a private array.  The line lies where waves would begin to
+// wait for others to end (2816 waves with 48 entries, 2304 with 64, 1536 with
+// 96); us with the whole stack in LDS -> with the window:
+//   rays                                131072      180224      196608    1048576
+//   260 k triangles, 44    closest  189 -> 201  192 -> 204  192 -> 206  403 -> 317
+//   instances (48 entries)     any  151 -> 152  152 -> 154  193 -> 160  396 -> 305
+//   500 k triangles (48)   closest  132 -> 135  134 -> 138  156 -> 139  367 -> 291
+//                              any  155 -> 159  162 -> 162  207 -> 164  484 -> 336
+//   2 M triangles (48)     closest  224 -> 232  226 -> 236  262 -> 237  607 -> 473
+//                              any  252 -> 257  276 -> 278  297 -> 279  699 -> 488
+//   2.4 k long, nested     closest  141 -> 145  193 -> 156  195 -> 157  386 -> 269
+//   triangles (64)             any  125 -> 129  169 -> 139  172 -> 140  724 -> 749
+// (724 and 749 are the chain of node visits of one ray).  The window has 32
+// entries where 16 are left, which the compiler keeps in registers, and in the
+// any-hit kernels, whose registers leave room for 32 more; closest-hit kernels
+// of deeper stacks take 16 (64 entries, 1 M rays: 269 us against 313).
+//
+// The parked ray setup (pre_park) takes 1.75 KB of LDS per wave: any-hit kernels
+// of 32-entry stacks hold 4 waves per SIMD with it and 5 without, yet are faster
+// with it, also where no ray enters an instance (4 M any-hit rays, 79 k
+// triangles: 812 us against 824; Cornell box 278 against 288).
+constexpr uint32_t kCus = 256, kLdsBytes = 160u * 1024u;
+template <int kStack>
+constexpr uint32_t kLdsStackWaves = kCus * (kLdsBytes / ((kStack + kPreSlots) * kTraceBlock * 4u));
+static_assert(kLdsStackWaves<32> >= kTraceWaves, "stacks of 32 entries stay in LDS");
+
+template <bool kAny, bool kCount, bool kSphere, int kStack, int kWindow>
 __global__ __launch_bounds__(kTraceBlock) void k_trace(DevScene sc, const float4 *__restrict__ rays, uint32_t n,
                                                         uint32_t per, uint4 *__restrict__ hits,
                                                         uint32_t *__restrict__ occluded, uint2 *__restrict__ visits,
                                                         uint32_t *__restrict__ err)
 {
-    constexpr int kWindow = kDeep ? kTraceWindow : 0;
-    __shared__ uint32_t stack[(kDeep ? kTraceWindow : kStack) * kTraceBlock];
+    constexpr int kDeep = kWindow > 0 ? kStack - kWindow : 0;
+    __shared__ uint32_t stack[(kStack - kDeep) * kTraceBlock];
     __shared__ float pre_park[kPreSlots * kTraceBlock];
     const uint32_t lane = __lane_id();
     const uint64_t below = (1ull << lane) - 1ull;
     uint32_t cur = blockIdx.x * per;
     const uint32_t end = cur + per < n ? cur + per : n;
-    LaneScratch<kTraceBlock, kWindow, true, kDeep ? kStack - kTraceWindow : 0> ls{
-        stack, nullptr, nullptr, nullptr, (int)lane, nullptr, 0, 0, pre_park};
+    uint32_t deep[kDeep > 0 ? kDeep : 1];
+    LaneScratch<kTraceBlock, kWindow, true, kDeep> ls{
+        stack, nullptr, nullptr, nullptr, (int)lane, nullptr, 0, 0, pre_park, deep};
     Traversal<kAny ? kModeSkipBoundary : kModeAll, kAny, false, kCount, kSphere, kStack> tv;
     TraceCounters cnt{0, 0};
     uint32_t i = 0;
@@ -105,15 +129,18 @@ static int launch_one(const ymrt_scene *sc, const ymrt_ray *rays, uint32_t n, ym
         hipLaunchKernelGGL(kernel, grid, dim3(kTraceBlock), 0, s, sc->dev, reinterpret_cast<const float4 *>(rays), n,
                            per, reinterpret_cast<uint4 *>(hits), occ, reinterpret_cast<uint2 *>(visits), sc->d_error);
     };
-    constexpr bool kDeepStack = kStack > 32;
     const bool spheres = sc->dev.has_spheres;
-    if (kDeepStack && waves > kTraceShallowWaves) {
-        if (spheres) launch(&k_trace<kAny, kCount, true, kStack, kDeepStack>);
-        else launch(&k_trace<kAny, kCount, false, kStack, kDeepStack>);
-    } else {
-        if (spheres) launch(&k_trace<kAny, kCount, true, kStack, false>);
-        else launch(&k_trace<kAny, kCount, false, kStack, false>);
+    if constexpr (kStack > 32) {
+        constexpr int kWindow = kAny || kStack <= 48 ? 32 : 16;
+        if (waves > kLdsStackWaves<kStack>) {
+            if (spheres) launch(&k_trace<kAny, kCount, true, kStack, kWindow>);
+            else launch(&k_trace<kAny, kCount, false, kStack, kWindow>);
+            YM_HIP(hipGetLastError());
+            return YMRT_OK;
+        }
     }
+    if (spheres) launch(&k_trace<kAny, kCount, true, kStack, 0>);
+    else launch(&k_trace<kAny, kCount, false, kStack, 0>);
     YM_HIP(hipGetLastError());
     return YMRT_OK;
 }
