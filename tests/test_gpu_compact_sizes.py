@@ -1,8 +1,9 @@
-"""Chunks of up to 65536 path slots are compacted by one launch, longer ones by
-three; up to 262144 paths share one shading launch, longer ones get one per
+"""Chunks of up to 65536 path slots are compacted by one launch; longer ones, and
+many of them in a batch (chunks times the square of the longest above 2^34), by
+three.  Up to 262144 paths share one shading launch, longer ones get one per
 class.  path_capacity sets the chunk, so the same frame runs through either;
 its image must not change, at chunks around a block's 1024 slots, the bound
-and odd pixel counts."""
+and odd pixel counts, nor that of a frame of a batch on either side."""
 import pytest
 
 import ymrt_amd
@@ -20,3 +21,19 @@ def test_chunk_sizes_keep_the_frame(gpu_ctx, w, h, spp):
         img, st = sc.render_frame(abi.render_settings(w, h, spp, 4, volume=1, path_capacity=cap), 2)
         assert st.chunks > 1 and torch.equal(img, ref), cap
     sc.close()
+
+
+@pytest.mark.parametrize("size,counts", [((256, 256), (4, 5)), ((128, 128), (64,)), ((144, 128), (40, 41))])
+def test_chunk_counts_keep_the_frames(gpu_ctx, size, counts):
+    """Batches whose rounds are compacted by one launch and by three."""
+    import torch
+    w, h = size
+    scene = [ymrt_amd.Scene(gpu_ctx, scenes.cornell_media(w, h, grid=False, halton_seed=s)) for s in range(3)]
+    rs = abi.render_settings(w, h, 1, 4, volume=1)
+    want = [sc.render_frame(rs, 2)[0] for sc in scene]
+    for count in counts:
+        jobs = [(scene[i % 3], rs, 2) for i in range(count)]
+        for i, (img, _) in enumerate(gpu_ctx.render_batch(jobs)):
+            assert torch.equal(img, want[i % 3]), (count, i)
+    for sc in scene:
+        sc.close()

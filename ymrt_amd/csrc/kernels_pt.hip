@@ -879,14 +879,20 @@ __global__ __launch_bounds__(kCompactThreads) void k_compact_scatter_m(const Fra
     compact_scatter_body<kMode>(f.prm, f.ps, pass, blockIdx.x);
 }
 
-// The whole compaction of a short chunk in one launch: a block gathers
+// The whole compaction of short chunks in one launch: a block gathers
 // kScanThreads slots and counts the matches before them itself.  The reads
-// grow with the square of the chunk, so this is for chunks of up to
-// kCompactSmall slots, where they are a few us while three launches of the
-// kernels above take about 23 with the gaps between them (Cornell 256x256 at 1
-// spp 2.11 -> 2.02 ms, a fixed-memory frame of 432 passes 51 -> 46; both run in
-// chunks of 65536 slots).
+// grow with the number of chunks and with the square of their length, so this
+// is for chunks of up to kCompactSmall slots and for launches of which the
+// chunks times the square of the longest is at most kCompactReads (32 MB of
+// flags read).  There the reads are a few us, while three launches of the
+// kernels above take about 23 with the gaps between them.  One launch against
+// three, ms per call, 1 spp: Cornell frames of 64x64, 128x128 and 256x256 1.26
+// and 1.40, 1.42 and 1.54, 1.65 and 1.72, with a medium (three compactions per
+// pass) 3.66 and 4.29, 4.22 and 4.86, 5.03 and 5.48; batches of them with the
+// medium, 4 and 16 of 256x256 8.32 and 8.79, 18.2 and 17.4; 64 of 256x256 49.6
+// and 44.8; 32 and 64 of 128x128 17.2 and 17.8, 28.2 and 28.1.
 constexpr uint32_t kCompactSmall = 65536;
+constexpr uint64_t kCompactReads = 1ull << 34;
 template <int kMode>
 __global__ __launch_bounds__(kScanThreads) void k_compact_small_m(const FrameSlot *__restrict__ fs, uint32_t pass)
 {
@@ -2140,8 +2146,9 @@ int launch_multi_medium(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v
 int launch_multi_compact(const FrameSlot *fs, uint32_t nfs, uint32_t blocks, uint32_t pass, int mode, hipStream_t s)
 {
     const dim3 g(blocks ? blocks : 1, nfs), b(kCompactThreads), g1(4, nfs), b1(kScanThreads);
-    // the longest chunk of the launch has at most blocks * kCompactSpan slots
-    if ((uint64_t)blocks * kCompactSpan <= kCompactSmall) {
+    // the longest chunk of the launch has at most this many slots
+    const uint64_t longest = (uint64_t)blocks * kCompactSpan;
+    if (longest <= kCompactSmall && nfs * longest * longest <= kCompactReads) {
         const dim3 gs(std::max(blocks, 1u) * (kCompactSpan / kScanThreads), nfs);
         if (mode == kCompactShade) hipLaunchKernelGGL(k_compact_small_m<kCompactShade>, gs, b1, 0, s, fs, pass);
         else if (mode == kCompactMedium) hipLaunchKernelGGL(k_compact_small_m<kCompactMedium>, gs, b1, 0, s, fs, pass);

@@ -39,6 +39,8 @@ constexpr int kTraceIdle = 3;
 //                              any  252 -> 257  276 -> 278  297 -> 279  699 -> 488
 //   2.4 k long, nested     closest  141 -> 145  193 -> 156  195 -> 157  386 -> 269
 //   triangles (64)             any  125 -> 129  169 -> 139  172 -> 140  724 -> 749
+//   16 k long, nested      closest 1533 ->1171 1852 ->1326 1966 ->1326 3509 ->2011
+//   triangles (96)             any  389 -> 280  423 -> 306  454 -> 307 1012 -> 547
 // (724 and 749 are the chain of node visits of one ray).  The window has 32
 // entries where 16 are left, which the compiler keeps in registers, and in the
 // any-hit kernels, whose registers leave room for 32 more; closest-hit kernels
