@@ -272,7 +272,10 @@ typedef struct ymrt_frame_stats {
     uint32_t passes;                 /* bounce passes launched                */
     uint32_t chunks;
     /* Per-stage GPU time measured with HIP events on the render stream (ms,
-     * summed over launches) and launch counts; filled when timing != 0. */
+     * summed over launches) and the kernels launched for it (shade, medium
+     * and transmit: with those that fill the stage's queue, one or three,
+     * and shade one for all classes of vertices or one per class); filled
+     * when timing != 0. */
     float ms_raygen, ms_extend, ms_shade, ms_shadow, ms_resolve;
     uint32_t launches_extend, launches_shade, launches_shadow;
     float ms_total;

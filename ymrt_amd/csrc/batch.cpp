@@ -40,9 +40,10 @@ int launch_multi_extend(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v
 int launch_multi_medium(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v, uint32_t waves, uint32_t pass,
                         hipStream_t s);
 // mode: 0 free flight, 1 shading, 2 transmittance
-int launch_multi_compact(const FrameSlot *fs, uint32_t nfs, uint32_t blocks, uint32_t pass, int mode, hipStream_t s);
+int launch_multi_compact(const FrameSlot *fs, uint32_t nfs, uint32_t blocks, uint32_t pass, int mode, hipStream_t s,
+                         uint32_t *launched);
 int launch_multi_shade(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v, uint64_t paths, uint32_t waves,
-                       uint32_t pass, hipStream_t s);
+                       uint32_t pass, hipStream_t s, uint32_t *launched);
 int launch_multi_shadow(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v, uint32_t waves, uint32_t pass,
                         hipStream_t s);
 int launch_multi_transmit(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v, uint32_t waves, uint32_t pass,
@@ -260,6 +261,7 @@ int render_batch(ymrt_context *ctx, const ymrt_batch_item *items, uint32_t n, ui
         YM_HIP(hipMemsetAsync(rb.counters, 0, sizeof(uint32_t) * kCountersPerSlot * nfs, stream));
         // one wave per 64 paths of the round, within the spill area
         uint64_t live = paths;  // no fewer than the paths still on their way
+        uint32_t launched = 0;  // not reported: frames share their launches
         const uint32_t waves = persistent_waves(paths, 0, rb.ps.spill_threads);
         const FrameSlot *fs = rb.slots;
         int rc;
@@ -268,14 +270,14 @@ int render_batch(ymrt_context *ctx, const ymrt_batch_item *items, uint32_t n, ui
         for (;;) {
             if ((rc = launch_multi_extend(fs, nfs, v, waves, pass, stream))) return rc;
             if (v.media) {
-                if ((rc = launch_multi_compact(fs, nfs, compact_blocks, pass, 0, stream))) return rc;
+                if ((rc = launch_multi_compact(fs, nfs, compact_blocks, pass, 0, stream, &launched))) return rc;
                 if ((rc = launch_multi_medium(fs, nfs, v, waves, pass, stream))) return rc;
             }
-            if ((rc = launch_multi_compact(fs, nfs, compact_blocks, pass, 1, stream))) return rc;
-            if ((rc = launch_multi_shade(fs, nfs, v, live, waves, pass, stream))) return rc;
+            if ((rc = launch_multi_compact(fs, nfs, compact_blocks, pass, 1, stream, &launched))) return rc;
+            if ((rc = launch_multi_shade(fs, nfs, v, live, waves, pass, stream, &launched))) return rc;
             if ((rc = launch_multi_shadow(fs, nfs, v, waves, pass, stream))) return rc;
             if (v.media) {
-                if ((rc = launch_multi_compact(fs, nfs, compact_blocks, pass, 2, stream))) return rc;
+                if ((rc = launch_multi_compact(fs, nfs, compact_blocks, pass, 2, stream, &launched))) return rc;
                 if ((rc = launch_multi_transmit(fs, nfs, v, waves, pass, stream))) return rc;
             }
             ++pass;

@@ -2143,7 +2143,9 @@ int launch_multi_medium(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v
     return YMRT_OK;
 }
 
-int launch_multi_compact(const FrameSlot *fs, uint32_t nfs, uint32_t blocks, uint32_t pass, int mode, hipStream_t s)
+// launched: counts the kernels it launches (so does launch_multi_shade).
+int launch_multi_compact(const FrameSlot *fs, uint32_t nfs, uint32_t blocks, uint32_t pass, int mode, hipStream_t s,
+                         uint32_t *launched)
 {
     const dim3 g(blocks ? blocks : 1, nfs), b(kCompactThreads), g1(4, nfs), b1(kScanThreads);
     // the longest chunk of the launch has at most this many slots
@@ -2154,6 +2156,7 @@ int launch_multi_compact(const FrameSlot *fs, uint32_t nfs, uint32_t blocks, uin
         else if (mode == kCompactMedium) hipLaunchKernelGGL(k_compact_small_m<kCompactMedium>, gs, b1, 0, s, fs, pass);
         else hipLaunchKernelGGL(k_compact_small_m<kCompactTransmit>, gs, b1, 0, s, fs, pass);
         YM_HIP(hipGetLastError());
+        *launched += 1;
         return YMRT_OK;
     }
     if (mode == kCompactShade) {
@@ -2170,6 +2173,7 @@ int launch_multi_compact(const FrameSlot *fs, uint32_t nfs, uint32_t blocks, uin
         hipLaunchKernelGGL(k_compact_scatter_m<kCompactTransmit>, g, b, 0, s, fs, pass);
     }
     YM_HIP(hipGetLastError());
+    *launched += 3;
     return YMRT_OK;
 }
 
@@ -2196,17 +2200,19 @@ constexpr uint64_t kShadeAllPaths = 1u << 18;
 
 // paths: no fewer than the launch's queues hold together.
 int launch_multi_shade(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v, uint64_t paths, uint32_t waves,
-                       uint32_t pass, hipStream_t s)
+                       uint32_t pass, hipStream_t s, uint32_t *launched)
 {
     if (v.graph && !v.media && !v.adj) {
         launch_persistent((k_shade_all_m<false, true>), waves, s, fs, nfs, pass);
         YM_HIP(hipGetLastError());
+        *launched += 1;
         return YMRT_OK;
     }
     if (paths <= kShadeAllPaths && !v.graph && !v.adj) {
         if (v.media) launch_persistent(k_shade_all_m<true>, waves, s, fs, nfs, pass);
         else launch_persistent(k_shade_all_m<false>, waves, s, fs, nfs, pass);
         YM_HIP(hipGetLastError());
+        *launched += 1;
         return YMRT_OK;
     }
     if (v.graph) v.adj ? shade_m<true, true>(fs, nfs, waves, pass, s) : shade_m<true, false>(fs, nfs, waves, pass, s);
@@ -2214,6 +2220,7 @@ int launch_multi_shade(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v,
     // volume vertices carry no adjoint events of their own
     if (v.media) launch_persistent((k_shade_m<true, false>), waves, s, fs, nfs, pass);
     YM_HIP(hipGetLastError());
+    *launched += v.media ? 4 : 3;
     return YMRT_OK;
 }
 

@@ -27,9 +27,10 @@ int launch_multi_extend(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v
 int launch_multi_medium(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v, uint32_t waves, uint32_t pass,
                         hipStream_t s);
 // mode: 0 free flight, 1 shading, 2 transmittance
-int launch_multi_compact(const FrameSlot *fs, uint32_t nfs, uint32_t blocks, uint32_t pass, int mode, hipStream_t s);
+int launch_multi_compact(const FrameSlot *fs, uint32_t nfs, uint32_t blocks, uint32_t pass, int mode, hipStream_t s,
+                         uint32_t *launched);
 int launch_multi_shade(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v, uint64_t paths, uint32_t waves,
-                       uint32_t pass, hipStream_t s);
+                       uint32_t pass, hipStream_t s, uint32_t *launched);
 int launch_multi_shadow(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v, uint32_t waves, uint32_t pass,
                         hipStream_t s);
 int launch_multi_transmit(const FrameSlot *fs, uint32_t nfs, const MultiVariant &v, uint32_t waves, uint32_t pass,
@@ -258,6 +259,7 @@ static int run_frame(ymrt_scene *sc, RenderBuffers *rb, uint32_t chunk_paths_max
         hipEvent_t a, b;
     };
     std::vector<Mark> marks;
+    uint32_t launches[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // kernels, by stage
     auto timed = [&](int stage, auto &&fn) -> int {
         hipEvent_t a = nullptr, b = nullptr;
         if (timing) {
@@ -290,18 +292,27 @@ static int run_frame(ymrt_scene *sc, RenderBuffers *rb, uint32_t chunk_paths_max
         uint32_t next_check = (uint32_t)rs->ray_depth + 1;
         uint64_t live = prm.chunk_paths;  // no fewer than the paths still on their way
         for (;;) {
+            ++launches[st(1)];
             if ((r = timed(st(1), [&] { return launch_multi_extend(f, 1, vv, waves, pass, stream); }))) return r;
             if (media && (r = timed(st(5), [&] {
-                              int q = launch_multi_compact(f, 1, blocks, pass, 0, stream);
+                              int q = launch_multi_compact(f, 1, blocks, pass, 0, stream, &launches[st(5)]);
+                              ++launches[st(5)];
                               return q ? q : launch_multi_medium(f, 1, vv, waves, pass, stream);
                           })))
                 return r;
-            if ((r = timed(st(2), [&] { return launch_multi_compact(f, 1, blocks, pass, 1, stream); }))) return r;
-            if ((r = timed(st(2), [&] { return launch_multi_shade(f, 1, vv, live, waves, pass, stream); })))
+            if ((r = timed(st(2), [&] {
+                     return launch_multi_compact(f, 1, blocks, pass, 1, stream, &launches[st(2)]);
+                 })))
                 return r;
+            if ((r = timed(st(2), [&] {
+                     return launch_multi_shade(f, 1, vv, live, waves, pass, stream, &launches[st(2)]);
+                 })))
+                return r;
+            ++launches[st(3)];
             if ((r = timed(st(3), [&] { return launch_multi_shadow(f, 1, vv, waves, pass, stream); }))) return r;
             if (media && (r = timed(st(6), [&] {
-                              int q = launch_multi_compact(f, 1, blocks, pass, 2, stream);
+                              int q = launch_multi_compact(f, 1, blocks, pass, 2, stream, &launches[st(6)]);
+                              ++launches[st(6)];
                               return q ? q : launch_multi_transmit(f, 1, vv, waves, pass, stream);
                           })))
                 return r;
@@ -376,12 +387,10 @@ static int run_frame(ymrt_scene *sc, RenderBuffers *rb, uint32_t chunk_paths_max
         stats->chunks = chunks;
         if (timing) {
             float ms[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-            uint32_t launches[8] = {0, 0, 0, 0, 0, 0, 0, 0};
             for (const Mark &m : marks) {
                 float t = 0.0f;
                 YM_HIP(hipEventElapsedTime(&t, m.a, m.b));
                 ms[m.stage] += t;
-                launches[m.stage]++;
             }
             stats->ms_raygen = ms[0];
             stats->ms_extend = ms[1];
@@ -394,9 +403,7 @@ static int run_frame(ymrt_scene *sc, RenderBuffers *rb, uint32_t chunk_paths_max
             stats->launches_transmit = launches[6];
             stats->ms_adjoint = ms[7];
             stats->launches_extend = launches[1];
-            // a pass of a scene with media counts its volume vertices as a
-            // launch of their own, also where they share one with the surfaces
-            stats->launches_shade = launches[2] + (media ? launches[1] : 0u);
+            stats->launches_shade = launches[2];
             stats->launches_shadow = launches[3];
             float tot = 0.0f;
             YM_HIP(hipEventElapsedTime(&tot, frame_a, frame_b));
