@@ -37,3 +37,19 @@ def test_chunk_counts_keep_the_frames(gpu_ctx, size, counts):
             assert torch.equal(img, want[i % 3]), (count, i)
     for sc in scene:
         sc.close()
+
+
+@pytest.mark.parametrize("w,h,spp", [(45, 31, 2), (331, 257, 4)])
+def test_graph_frames_in_one_shading_launch_and_by_class(gpu_ctx, w, h, spp):
+    """A frame with texture graphs and no media shades all classes in one launch,
+    in rounds shared with a medium it takes one per class."""
+    import torch
+    graph = ymrt_amd.Scene(gpu_ctx, scenes.textured_box(w, h))
+    fog = ymrt_amd.Scene(gpu_ctx, scenes.cornell_media(64, 48, grid=False))
+    rs, rf = abi.render_settings(w, h, spp, 5), abi.render_settings(64, 48, 1, 5, volume=1)
+    want, st = graph.render_frame(rs, 3, timing=True)
+    assert st.launches_shade == (1 if w * h * spp < 65536 else 3) * st.passes + st.passes
+    (img, _), (mist, _) = gpu_ctx.render_batch([(graph, rs, 3), (fog, rf, 3)])
+    assert torch.equal(img, want) and torch.equal(mist, fog.render_frame(rf, 3)[0])
+    graph.close()
+    fog.close()
