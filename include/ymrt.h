@@ -253,7 +253,7 @@ typedef struct ymrt_render_settings {
     float exposure;
     uint32_t path_capacity;          /* paths in flight per chunk; 0: up to 64 M,
                                         within a quarter of free device memory
-                                        (at most 720 B per path)              */
+                                        (589 B per path)                      */
     uint32_t persistent_waves;       /* waves of each persistent pass kernel,
                                         at most 5120 (the traversal spill
                                         area); 0: one per 64 paths of the

@@ -7,6 +7,7 @@
 #include <memory>
 #include <vector>
 
+#include "../../ymrt_amd/csrc/buffers.hpp"
 #include "../../ymrt_amd/csrc/bvh.hpp"
 #include "../../ymrt_amd/csrc/dev_traverse.hpp"
 
@@ -164,4 +165,6 @@ void ht_visit(const void *nodes, const float *rays, uint32_t n, int park, uint32
         while (tv.sp > 0) *o++ = s->ls.pop(--tv.sp);
     }
 }
+
+uint64_t ht_path_bytes() { return path_bytes(); }
 }

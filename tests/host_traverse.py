@@ -1,5 +1,5 @@
 """The library's traversal compiled for the host (tests/host/traverse.cpp), for
-scenes of one mesh under one instance."""
+scenes of one mesh under one instance, and the path state's size."""
 import ctypes as C
 import os
 import subprocess
@@ -28,6 +28,7 @@ def lib():
         L.ht_trace.restype = C.c_int
         L.ht_trace.argtypes = [vp, vp, u32, C.c_int, C.c_int, vp, vp]
         L.ht_visit.argtypes = [vp, vp, u32, C.c_int, vp]
+        L.ht_path_bytes.restype = C.c_uint64
         _lib = L
     return _lib
 

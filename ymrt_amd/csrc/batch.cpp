@@ -54,7 +54,6 @@ int launch_multi_resolve(const FrameSlot *fs, uint32_t nfs, uint32_t pixel_block
 // Same sizing rule as a single frame (render.cpp): up to 64 M paths in
 // flight, within a quarter of the free device memory.
 constexpr uint64_t kBatchCapacity = 1ull << 26;
-constexpr uint64_t kBatchPathBytes = 720;
 
 namespace {
 
@@ -164,7 +163,7 @@ int render_batch(ymrt_context *ctx, const ymrt_batch_item *items, uint32_t n, ui
     if (cap > held) {
         size_t free_b = 0, total_b = 0;
         YM_HIP(hipMemGetInfo(&free_b, &total_b));
-        cap = std::min<uint64_t>(cap, ((uint64_t)free_b + held * kBatchPathBytes) / 4 / kBatchPathBytes);
+        cap = std::min<uint64_t>(cap, ((uint64_t)free_b + held * path_bytes()) / 4 / path_bytes());
     }
     cap = std::max<uint64_t>(std::max<uint64_t>(cap, spp_max), std::min<uint64_t>(held, kBatchCapacity));
     YM_REQUIRE(cap <= 0xFFFFFFFFull, "batch capacity overflow");

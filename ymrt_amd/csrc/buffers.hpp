@@ -83,4 +83,21 @@ inline int layout_buffers(RenderBuffers &rb, size_t n, uint32_t spill_threads, G
     return rc;
 }
 
+// Device memory that each path of a frame chunk takes (rounded up), with what
+// the adjoint's replay adds when it first runs.
+inline uint64_t path_bytes()
+{
+    auto total = [](size_t n) {
+        RenderBuffers sizes;  // owns nothing: only the layout is computed
+        size_t bytes = 0;
+        layout_buffers(sizes, n, 0, [&](auto *&p, size_t count) {
+            bytes += sizeof(*p) * count;
+            return 0;
+        });
+        return bytes;
+    };
+    constexpr size_t n = (size_t)kCompactSpan * 256;
+    return (total(n) - total(0) + n - 1) / n + sizeof(*PathState{}.adj_g);
+}
+
 }  // namespace ym

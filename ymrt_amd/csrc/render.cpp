@@ -42,11 +42,10 @@ int launch_multi_resolve(const FrameSlot *fs, uint32_t nfs, uint32_t pixel_block
 // chunk ends in passes that hold only a frame's longest paths, where the GPU
 // idles; larger chunks amortise those tails (interior 1080p x 64 spp: 1417
 // ms per frame in 4 M-path chunks, 1188 in 16 M, 1129 in 64 M).  The path
-// state costs about kPathBytes per path, so a chunk is also held to a quarter
+// state costs path_bytes() per path, so a chunk is also held to a quarter
 // of the device memory free when the buffers are first allocated, and never
 // to more than the frame needs.
 constexpr uint32_t kDefaultCapacity = 1u << 26;
-constexpr uint64_t kPathBytes = 720;
 
 void destroy_render_buffers(ymrt_scene *sc)
 {
@@ -180,8 +179,8 @@ int render_frame_with(ymrt_scene *sc, RenderBuffers *&buffers, const ymrt_render
             // this call would give back), never below what it already holds
             size_t free_b = 0, total_b = 0;
             YM_HIP(hipMemGetInfo(&free_b, &total_b));
-            const uint64_t held = buffers ? (uint64_t)buffers->cap * kPathBytes : 0;
-            cap = std::min<uint64_t>(want, (free_b + held) / 4 / kPathBytes);
+            const uint64_t held = buffers ? (uint64_t)buffers->cap * path_bytes() : 0;
+            cap = std::min<uint64_t>(want, (free_b + held) / 4 / path_bytes());
             if (buffers) cap = std::max<uint64_t>(cap, buffers->cap);
         }
         cap = std::max<uint64_t>(cap, spp);
