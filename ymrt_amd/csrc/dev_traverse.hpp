@@ -223,7 +223,7 @@ YM_HD int tri_hit_back(const DevScene &sc, uint32_t inst, uint32_t tri, f3 d)
 // With kPreSlots, the world-space ray setup (reciprocal direction, shear
 // constants and axis) is parked in LDS [kPreSlots][kBlock] when a traversal
 // enters an instance and read back when it leaves, instead of being
-// recomputed with six divisions.
+// recomputed with five divisions.
 //
 // With kDeep > 0 the deeper entries go to a private array of kDeep instead of
 // the spill area (for kernels that own no memory).  The kernel declares the
@@ -238,7 +238,8 @@ struct LaneScratch {
     uint32_t *stack;        // [kWindow or kStack][kBlock]
     uint32_t *nb_prim;      // [kNearbyCap][kBlock]
     float *nb_t;
-    int *nb_back;           // during a traversal the side code (side_code), after resolve_backs the side
+    int *nb_back;           // during a traversal the crossing's code (Traversal::ex_code), after
+                            // resolve_backs the side
     int lane;
     uint32_t *spill;        // global [kMaxSpill][spill_stride], unused when kWindow == 0
     uint32_t spill_stride, spill_index;
@@ -355,7 +356,6 @@ struct TraceCounters {
 // then; it costs registers in the traversal loop).
 constexpr int kTravContinue = 0, kTravHit = 1, kTravMiss = 2, kTravOverflow = -1;
 
-//
 // Which side of a triangle a ray meets takes a normalised normal (about 70
 // instructions), and a traversal with the nearby list would need it for every
 // triangle the ray crosses, in steps where few lanes of the wave are at a

@@ -11,11 +11,12 @@
 //           media are on), adds the NEE term in the reference's order
 //   resolve per-pixel mean over the samples of the chunk (sample order fixed,
 //           so frames are deterministic -- no float atomics)
-// Path state is SoA in HBM indexed by the path's slot; queues hold slot ids
-// and are compacted per wave64 with a ballot + one atomic per wave.  Every
-// kernel deals its queue over its waves from the length in a device counter,
-// so launches never need the host to know queue lengths (no host round trip
-// per stage).
+// Path state lies in HBM in records indexed by the path's slot (PathState);
+// queues hold slot ids and are filled per wave64 with a ballot + one atomic per
+// fetch of items, or by the compaction of the slots' stage flags.  Every kernel
+// deals its queue over its waves from the length in a device counter, so
+// launches never need the host to know queue lengths (no host round trip per
+// stage).
 #include <algorithm>
 #include <mutex>
 #include <unordered_map>
@@ -78,8 +79,8 @@ struct Share {
 // Persistent loop over n items (one wave per block): body(i, p, out) handles
 // item i < n, sets p (the path slot it appends) and out[q] for each output
 // queue q.  stage: LDS of kQueues * kS * 64 words.  Survivors of a fetch's
-// sub-batches (at most kS) are staged in LDS and then published with one atomic per queue and
-// a coalesced copy.
+// sub-batches (at most kS) are staged in LDS and then published with one atomic
+// per queue and a coalesced copy.
 template <int kQueues, int kS = kSub, typename Body>
 __device__ __forceinline__ void run_items(uint32_t *stage, const Share &share, uint32_t *fetch, uint32_t n,
                                           uint32_t *const *counters, uint32_t *const *queues, Body &&body)
@@ -320,10 +321,11 @@ __device__ __forceinline__ uint32_t *pass_work(const FrameSlot &f, uint32_t pass
 //   * kMaxGrain when every wave of the grid gets that many: long queues, whose
 //     fetch atomics (tens of ns each on one address, one after another across
 //     the chip) would set the pace in smaller shares;
-//   * down to kMinGrain, one full wave, otherwise, so that a short queue is spread over all
-//     the waves the GPU holds: a wave's items run one sub-batch after another,
-//     each a chain of dependent loads, and with shares of kMaxGrain a
-//     65536-path launch would occupy 256 of 1024 SIMDs for four such chains.
+//   * down to kMinGrain, one full wave, otherwise, so that a short queue is
+//     spread over all the waves the GPU holds: a wave's items run one sub-batch
+//     after another, each a chain of dependent loads, and with shares of
+//     kMaxGrain a 65536-path launch would occupy 256 of 1024 SIMDs for four
+//     such chains.
 //     Shares of less than a wave (16 or 32 rays to each traversal wave, on
 //     more waves) are slower: the SIMDs then issue more instructions for the
 //     same rays (Cornell 256x256 at 1 spp 2.9 and 2.4 ms against 2.1).
@@ -331,10 +333,11 @@ __device__ __forceinline__ uint32_t *pass_work(const FrameSlot &f, uint32_t pass
 // one round of shares covers takes no atomics at all; waves without a share
 // leave at once.  rot: the grid index of the first wave that takes a share; the
 // waves used come back, so that a kernel with several queues can deal each to
-// other waves.  Measured against shares of kMaxGrain from one counter (with
-// 16-ray shares in the traversal kernels): Cornell 256x256 at 1 spp 6.9 -> 3.1 ms, its 512x512 smoke at 16 spp (23
-// passes, the last of them short) 49 -> 40 ms, the interior at 1080p and 1 spp
-// 27.7 -> 24.1 ms, at 64 spp 958 -> 950 ms.
+// other waves.  Shares of kMaxGrain from one counter against these (measured
+// when the traversal kernels still took 16 rays to a wave, which cost Cornell
+// 2.9 ms where it now takes 2.1): Cornell 256x256 at 1 spp 6.9 -> 3.1 ms, its
+// 512x512 smoke at 16 spp (23 passes, the last of them short) 49 -> 40 ms, the
+// interior at 1080p and 1 spp 27.7 -> 24.1 ms, at 64 spp 958 -> 950 ms.
 template <uint32_t kMinGrain, uint32_t kMaxGrain, typename Count, typename Work, typename Body>
 __device__ __forceinline__ uint32_t for_slots(const FrameSlot *__restrict__ fs, uint32_t nfs, Count count, Work work,
                                               Body body, uint32_t rot = 0)
@@ -1594,10 +1597,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kGraph ?
     shade_class<kVolume, kGraph, kClass, kAdj>(ShadeLds{stage, tex_stk, adj_lds}, fs, nfs, pass, 0);
 }
 
-// All shading classes of a pass of short queues in one launch, and with kMedia
-// the volume vertices.  Launched one after another, each class is a chain of
-// dependent loads of 25-35 us on a queue that leaves most of the GPU idle;
-// here a class' waves are others than those the classes before it took.
+// All shading classes of a pass in one launch, and with kMedia the volume
+// vertices: for short queues and for frames with texture graphs
+// (launch_multi_shade).  Launched one after another, each class is a chain of
+// dependent loads of 25-35 us, on a short queue with most of the GPU idle; here
+// a class' waves are others than those the classes before it took.
 template <bool kMedia, bool kGraph = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kGraph ? 2 : 3))) void k_shade_all_m(const FrameSlot *__restrict__ fs, uint32_t nfs, uint32_t pass)
 {
@@ -2185,17 +2189,24 @@ static void shade_m(const FrameSlot *fs, uint32_t nfs, uint32_t waves, uint32_t 
     launch_persistent((k_shade_m<false, kGraph, kMatMetal, kAdj>), waves, s, fs, nfs, pass);
 }
 
-// With up to this many paths the shading classes share one launch (not in the
-// adjoint's replay, nor in frames with texture graphs and media).  One launch against one
-// per class, ms per frame at 2^16, 2^18, 2^19 and 2^21 paths: Cornell 1.64 and
-// 2.01, 2.94 and 3.34, 4.56 and 4.89, 8.92 and 8.97; outdoor with fog 3.13 and
-// 4.21, 4.97 and 5.98, 6.59 and 7.39, 12.9 and 12.8; smoke 5.48 and 6.67, 8.21
-// and 9.26, 11.4 and 11.9, 28.9 and 27.4; interior 3.89 and 4.22, 6.24 and
-// 6.47, 10.6 and 10.0, 21.1 and 20.6.  Long queues lose: their waves run
-// different classes at once, which share an instruction cache.  Frames with
-// texture graphs and no media share one launch at any length: their general
-// class takes most of the time, and the others then fill the lanes and waves
-// it leaves at its end (procedural box, 4.9 M paths: 17.8 -> 17.2 ms).
+// With up to this many paths the shading classes share one launch (not in
+// frames with texture graphs and media, nor in the adjoint's replay, for which
+// no such kernel is built).  One launch against one per class, ms per frame at
+// 2^16, 2^18, 2^19 and 2^21 paths: Cornell 1.64 and 2.01, 2.94 and 3.34, 4.56
+// and 4.89, 8.92 and 8.97; outdoor with fog 3.13 and 4.21, 4.97 and 5.98, 6.59
+// and 7.39, 12.9 and 12.8; smoke 5.48 and 6.67, 8.21 and 9.26, 11.4 and 11.9,
+// 28.9 and 27.4; interior 3.89 and 4.22, 6.24 and 6.47, 10.6 and 10.0, 21.1 and
+// 20.6.  Long queues lose: their waves run different classes at once, which
+// share an instruction cache.
+// Frames with texture graphs and no media share one launch at any length: all
+// their classes run at 2 waves per SIMD, and one class' waves fill what another
+// leaves at its end.  At 2^16, 2^18, 0.8 M, 2.1 M and 4.2 M paths: Cornell with a
+// checkerboard 1.66 and 2.08, 3.06 and 3.46, 5.17 and 5.54, 7.48 and 7.85, 13.8
+// and 14.3; the interior with one graph-textured object 3.18 and 3.43, 5.23 and
+// 5.56, 9.10 and 9.67, 15.6 and 17.2, 25.8 and 27.2; a batch of six such rooms
+// without and one small frame with a graph 39.8 and 42.2.  A box whose every
+// wall runs a graph is the exception, between 2^18 and 2^21 paths: 1.84 and
+// 2.18, 3.57 and 3.51, 6.99 and 6.52, 10.8 and 10.7, 20.9 and 21.8.
 constexpr uint64_t kShadeAllPaths = 1u << 18;
 
 // paths: no fewer than the launch's queues hold together.
